@@ -48,8 +48,15 @@ const KernelName kKernels[] = {
     {K_GEMM_REDUCE, "gh_gemm_reduce"},     {K_GEMM_TAIL, "gh_gemm_tail"},
     {K_GEMM_REDUCE_SWIGLU, "gh_gemm_reduce_swiglu"},
     {K_GEMM3_MIXED_R128, "gh_gemm3_mixed_r128"},
-    {K_GEMM_REDUCE_SEG, "gh_gemm_reduce_seg"},     {K_ATTN_PREFILL_G4, "gh_attn_prefill_g4"},
-    {K_ATTN_PREFILL_G4_R16, "gh_attn_prefill_g4_r16"},
+    {K_GEMM_REDUCE_SEG, "gh_gemm_reduce_seg"},     {K_ATTN_MERGE, "gh_attn_merge"},
+    {K_ATTN_PREFILL_G1, "gh_attn_prefill_g1"}, {K_ATTN_PREFILL_G1_R16, "gh_attn_prefill_g1_r16"},
+    {K_ATTN_PREFILL_G1_R16_K, "gh_attn_prefill_g1_r16_k"},
+    {K_ATTN_PREFILL_G2, "gh_attn_prefill_g2"}, {K_ATTN_PREFILL_G2_R16, "gh_attn_prefill_g2_r16"},
+    {K_ATTN_PREFILL_G2_R16_K, "gh_attn_prefill_g2_r16_k"},
+    {K_ATTN_PREFILL_G4, "gh_attn_prefill_g4"}, {K_ATTN_PREFILL_G4_R16, "gh_attn_prefill_g4_r16"},
+    {K_ATTN_PREFILL_G4_R16_K, "gh_attn_prefill_g4_r16_k"},
+    {K_ATTN_PREFILL_G8, "gh_attn_prefill_g8"}, {K_ATTN_PREFILL_G8_R16, "gh_attn_prefill_g8_r16"},
+    {K_ATTN_PREFILL_G8_R16_K, "gh_attn_prefill_g8_r16_k"},
     {K_GEMM3_Q4K_R128, "gh_gemm3_q4k_r128"},   {K_GEMM3_Q6K_R128, "gh_gemm3_q6k_r128"},
     {K_GEMM3_Q4K_R96, "gh_gemm3_q4k_r96"},     {K_GEMM3_Q6K_R96, "gh_gemm3_q6k_r96"},
     {K_TOPK_PARTIAL, "gh_topk_partial"},       {K_TOPK_FINAL, "gh_topk_final"},
@@ -310,29 +317,82 @@ int ensure_counters(gh_backend* b, size_t slots) {
     return GH_OK;
 }
 
-// Causal GQA attention for `rows` query rows at positions base + r (+ *pos_ptr);
-// max_pos bounds the positions the launch can see (sizes the split grid).
-constexpr uint32_t kAttnPrefillMinRows = 32;
+// Key splits of a prefill attention launch of `wgs` 16-row workgroups whose longest query block
+// has `tiles` key tiles (gh_set_attention_splits replaces the policy's count). A workgroup takes
+// about 1.05 us per 64-key tile whatever its rows (the tile's dependent chain), the partials and
+// their merge 3-4 us, so a launch splits when that saves at least four tiles, into about 1.5
+// workgroups per CU. G = 4, 8 kv heads, us with 1 split and with this count: 5 rows at 8000
+// 133.1 / 14.0 (32), 32 rows at 4000 68.8 / 15 (12), 100 rows at 4000 70.5 / 27 (6), 256 rows at
+// 1000 24.6 / 22.6 (3); where it stays at one: 100 rows at 0 5.5 (9.0 with two), 256 rows at 0
+// 7.7 (12.2).
+static uint32_t prefill_splits(const gh_backend* b, uint32_t wgs, uint32_t tiles) {
+    if (b->attn_splits) return std::min({b->attn_splits, tiles, 32u});
+    const uint32_t s = std::max<uint32_t>(1, std::min<uint32_t>({b->cus * 3 / 2 / wgs, tiles, 32u}));
+    return tiles - ceil_div(tiles, s) >= 4 ? s : 1;
+}
+
+// Attention of `rows` >= 2 query rows at positions base + r on the matrix cores, 1, 2, 4 or 8
+// query heads per kv head: 32 query rows per wave where that gives every CU a workgroup (K/V
+// tiles shared by twice the rows of 16-row blocks; 248 VGPRs keep two workgroups resident per
+// CU), else 16, and key splits with a merge launch where the query blocks leave CUs idle.
+static int attention_prefill(gh_backend* b, GhAttnArgs a, uint32_t group) {
+    const uint32_t hw = std::min(group, 4u), ng = a.q_heads / hw;
+    const uint32_t rw = 4 / hw;  // row groups per workgroup
+    const int first = group == 1   ? K_ATTN_PREFILL_G1
+                      : group == 2 ? K_ATTN_PREFILL_G2
+                      : group == 4 ? K_ATTN_PREFILL_G4
+                                   : K_ATTN_PREFILL_G8;
+    a.splits = 1;
+    if ((uint64_t)ceil_div(a.rows, 32 * rw) * ng >= b->cus)
+        return launch(b, (GhKernel)first, ceil_div(a.rows, 32 * rw), ng, 1, 256, &a);
+    const uint32_t pq = 16 * rw, nqb = ceil_div(a.rows, pq);
+    uint32_t splits = prefill_splits(b, nqb * ng, ceil_div(a.base + a.rows, 64));
+    if (splits > 1) {
+        const size_t n = (size_t)a.rows * a.q_heads * splits;
+        const int rc = ensure_workspace(b, attention_workspace(a.rows, a.q_heads, splits));
+        if (rc == GH_E_OOM) {  // no room for the partials: one split
+            (void)hipGetLastError();
+            b->err.clear();
+            splits = 1;
+        } else if (rc) {
+            return rc;
+        }
+        char* ws = (char*)b->ws + kArgmaxBytes;
+        a.part_m = (uint64_t)ws;
+        a.part_l = (uint64_t)(ws + n * 4);
+        a.part_acc = (uint64_t)(ws + n * 8);
+    }
+    if (splits == 1) return launch(b, (GhKernel)(first + 1), nqb, ng, 1, 256, &a);
+    a.splits = splits;
+    const int rc = launch(b, (GhKernel)(first + 2), nqb, ng, splits, 256, &a);
+    if (rc) return rc;
+    a.pad = pq;
+    return launch(b, K_ATTN_MERGE, ceil_div((uint64_t)a.rows * a.q_heads, 4), 1, 1, 256, &a);
+}
 
 int op_attention(gh_backend* b, const gh_buf* out, const gh_buf* q, const gh_kv* kv,
                  uint32_t q_heads, uint32_t base, uint32_t rows, uint32_t layer,
                  const void* pos_ptr, uint32_t max_pos, const AttnScratch* fixed) {
     const uint32_t group = q_heads / kv->kv_heads;
-    // the XCD-local split merge when the start-up probe confirmed the dispatch rule it needs
-    const bool xl = b->attn_xcd_merge && b->xcds != 0;
-    GhKernel k;
-    switch (group) {
-        case 1: k = xl ? K_ATTN_G1_X : K_ATTN_G1; break;
-        case 2: k = xl ? K_ATTN_G2_X : K_ATTN_G2; break;
-        // four or eight query heads per kv head: the matrix-core decode (the K and value dims
-        // are 128, which check_attention and the model enforce)
-        case 4: k = xl ? K_ATTN_MFMA_G4_X : K_ATTN_MFMA_G4; break;
-        case 8: k = xl ? K_ATTN_MFMA_G8_X : K_ATTN_MFMA_G8; break;
-        default: return fail(b, GH_E_UNSUPPORTED, "attention: GQA group must be 1, 2, 4 or 8");
+    if (group != 1 && group != 2 && group != 4 && group != 8)
+        return fail(b, GH_E_UNSUPPORTED, "attention: GQA group must be 1, 2, 4 or 8");
+    // decode reads a layer's K/V through 32-bit buffer ranges and takes the head counts and the
+    // launch's rows as 16-bit fields; the limits hold for every call that it may serve, and for
+    // the other groups' chunks, as before the prefill kernels took those
+    if (pos_ptr || rows < 32 || group != 4) {
+        if (((uint64_t)kv->context + 2048) * kv->kv_heads * kv->head_dim * 2 >= (1ull << 31))
+            return fail(b, GH_E_UNSUPPORTED, "attention: a layer's K or V cache of 2 GiB or more");
+        if (q_heads > 0xFFFFu || kv->kv_heads > 0xFFFFu)
+            return fail(b, GH_E_UNSUPPORTED, "attention: more than 65535 heads");
     }
-    // Batched prefill on the matrix cores: 32-row query blocks x kv heads (G = 4, head 128).
-    if (!pos_ptr && rows >= kAttnPrefillMinRows && group == 4 && kv->head_dim == 128 &&
-        kv->value_dim == 128) {
+    // Several rows: the prefill kernels, except where the decode kernels, which read each row's
+    // K/V again, have so little to read that the missing merge launch counts (G = 4, 8 kv heads,
+    // decode against prefill: 2 rows at 300 6.4 / 6.8 us, 5 at 300 6.6 / 7.1, 16 at 0 3.9 / 4.4;
+    // 5 at 1000 9.8 / 7.9, 16 at 300 8.2 / 8.0; G = 8, whose decode rows cost more: 2 rows at 300
+    // 8.1 / 6.9, 16 at 0 3.8 / 4.4)
+    const uint64_t reads = (uint64_t)rows * (base + rows) * kv->kv_heads;
+    const bool few = rows < 32 && reads <= (group == 8 ? 4096u : 16384u);
+    if (!pos_ptr && rows > 1 && !few) {
         GhAttnArgs a{};
         a.q = q->addr;
         a.kc = kv->k.addr;
@@ -347,23 +407,23 @@ int op_attention(gh_backend* b, const gh_buf* out, const gh_buf* q, const gh_kv*
         a.base = base;
         a.rows = rows;
         a.scale = 1.0f / std::sqrt((float)kv->head_dim);
-        // 32 query rows per workgroup (K/V tiles shared by twice the rows of 16-row blocks;
-        // 248 VGPRs keep two workgroups resident per CU), 16 when 32-row blocks would leave
-        // CUs without a workgroup
-        if ((uint64_t)ceil_div(rows, 32) * kv->kv_heads < b->cus)
-            return launch(b, K_ATTN_PREFILL_G4_R16, ceil_div(rows, 16), kv->kv_heads, 1, 256, &a);
-        return launch(b, K_ATTN_PREFILL_G4, ceil_div(rows, 32), kv->kv_heads, 1, 256, &a);
+        return attention_prefill(b, a, group);
     }
-    // decode reads a layer's K/V through 32-bit buffer ranges
-    if (((uint64_t)kv->context + 2048) * kv->kv_heads * kv->head_dim * 2 >= (1ull << 31))
-        return fail(b, GH_E_UNSUPPORTED, "attention: a layer's K or V cache of 2 GiB or more");
+    // the XCD-local split merge when the start-up probe confirmed the dispatch rule it needs
+    const bool xl = b->attn_xcd_merge && b->xcds != 0;
+    GhKernel k;
+    switch (group) {
+        case 1: k = xl ? K_ATTN_G1_X : K_ATTN_G1; break;
+        case 2: k = xl ? K_ATTN_G2_X : K_ATTN_G2; break;
+        // four or eight query heads per kv head: the matrix-core decode (the K and value dims
+        // are 128, which check_attention and the model enforce)
+        case 4: k = xl ? K_ATTN_MFMA_G4_X : K_ATTN_MFMA_G4; break;
+        default: k = xl ? K_ATTN_MFMA_G8_X : K_ATTN_MFMA_G8; break;
+    }
     const uint32_t splits = attention_splits(b, max_pos + 1, kv->kv_heads, rows);
     // the merge of a launch of at most 16 splits reads 16 slots (same bits, half the loads)
     if (k == K_ATTN_MFMA_G4 && splits <= 16) k = K_ATTN_MFMA_G4_S16;
     if (k == K_ATTN_MFMA_G4_X && splits <= 16) k = K_ATTN_MFMA_G4_S16_X;
-    // the kernels take the head counts and the launch's rows as 16-bit fields
-    if (q_heads > 0xFFFFu || kv->kv_heads > 0xFFFFu)
-        return fail(b, GH_E_UNSUPPORTED, "attention: more than 65535 heads");
     char* ws = nullptr;
     void* counters = nullptr;
     uint32_t group_rows = rows;

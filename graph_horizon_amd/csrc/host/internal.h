@@ -67,8 +67,19 @@ enum GhKernel : int {
     K_GEMM_REDUCE_SWIGLU,
     K_GEMM3_MIXED_R128,
     K_GEMM_REDUCE_SEG,
+    K_ATTN_PREFILL_G1,  // each followed by its 16-row form, without and with key splits
+    K_ATTN_PREFILL_G1_R16,
+    K_ATTN_PREFILL_G1_R16_K,
+    K_ATTN_PREFILL_G2,
+    K_ATTN_PREFILL_G2_R16,
+    K_ATTN_PREFILL_G2_R16_K,
     K_ATTN_PREFILL_G4,
     K_ATTN_PREFILL_G4_R16,
+    K_ATTN_PREFILL_G4_R16_K,
+    K_ATTN_PREFILL_G8,
+    K_ATTN_PREFILL_G8_R16,
+    K_ATTN_PREFILL_G8_R16_K,
+    K_ATTN_MERGE,
     K_GEMM3_Q4K_R128,
     K_GEMM3_Q6K_R128,
     K_GEMM3_Q4K_R96,

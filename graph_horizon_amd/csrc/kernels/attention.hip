@@ -581,12 +581,13 @@ GH_KERNEL __launch_bounds__(64) void gh_xcd_probe(uint64_t out, uint32_t gx, uin
 }
 
 // ---------------------------------------------------------------------------------------------
-// Causal GQA prefill attention on the matrix cores (flash attention, G = 4 query heads per kv
-// head, head_dim = value_dim = 128).
+// Causal GQA attention of several query rows on the matrix cores (flash attention, G = 1, 2, 4
+// or 8 query heads per kv head, head_dim = value_dim = 128): prefill chunks of 2 rows and more.
 //
-// Grid (query blocks of 16·QT rows, kv heads), 256 threads; wave w owns query head 4·kvh + w
-// for the block's rows, so every K/V tile staged in LDS serves all four heads. Per tile of 64
-// key positions, with v_mfma_f32_16x16x32_f16 and FP32 accumulators:
+// Grid (query blocks, groups of HW = min(G, 4) query heads of one kv head, key splits), 256
+// threads. Wave w owns query head w % HW of its group and the row group w / HW of the block
+// (4 / HW row groups of 16·QT rows), so every K/V tile staged in LDS serves all four waves. Per
+// tile of 64 key positions, with v_mfma_f32_16x16x32_f16 and FP32 accumulators:
 //   S^T = K · Q^T   A = K rows (LDS), B = the wave's FP16 query rows (registers); the output
 //                   layout gives each lane one query row (lane % 16) and four key positions
 //                   per 16 x 16 tile, so the row's running max/sum stay in that lane;
@@ -597,6 +598,9 @@ GH_KERNEL __launch_bounds__(64) void gh_xcd_probe(uint64_t out, uint32_t gx, uin
 // Softmax in base 2: scores are scaled by scale·log2(e), p = 2^(s - m), rescale 2^(m_old - m).
 // Rows: query r at position base + r attends positions 0..base + r (the reference's prefill,
 // attention/mod.rs:582-725). Query blocks run heaviest (latest) first.
+// Key splits (a.splits > 1): where the query blocks alone leave CUs idle (few rows), split z of
+// a block takes its key tiles z·per .. + per, per = ceil(the last block's tiles / splits), and
+// writes (m, l, unnormalized acc) as FP32 partials that gh_attn_merge combines.
 namespace {
 typedef _Float16 ah8 __attribute__((ext_vector_type(8)));
 typedef float af4 __attribute__((ext_vector_type(4)));
@@ -684,9 +688,19 @@ struct Flag {
 typedef float af2 __attribute__((ext_vector_type(2)));
 typedef _Float16 ah2 __attribute__((ext_vector_type(2)));
 
-template <int QT>  // query tiles of 16 rows per wave
-__device__ __forceinline__ void attn_prefill_g4(const GhAttnArgs& a) {
-    constexpr uint32_t kPQ = 16 * QT;  // query rows per workgroup
+// key tiles of query block qb (PQ rows per block); every split of a launch takes
+// ceil(tiles of the last block / splits) of them
+__device__ __forceinline__ uint32_t attn_tiles(const GhAttnArgs& a, uint32_t qb, uint32_t pq) {
+    return (a.base + min((qb + 1) * pq, a.rows) + kPK - 1) / kPK;
+}
+
+// QT: query tiles of 16 rows per wave; G: query heads per kv head; SPLIT: key splits (the plain
+// form carries none of their branches: with them at run time, 2048 rows of G = 4 took 69 us
+// instead of 58)
+template <int QT, int G, bool SPLIT>
+__device__ __forceinline__ void attn_prefill(const GhAttnArgs& a) {
+    constexpr uint32_t HW = G < 4 ? G : 4, RW = 4 / HW;  // heads and row groups per workgroup
+    constexpr uint32_t kPQ = 16 * QT * RW;               // query rows per workgroup
     __shared__ __attribute__((aligned(16))) _Float16 kt[2][kPK * 128];
     __shared__ __attribute__((aligned(16))) _Float16 vt[2][kPK * 128];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -695,12 +709,19 @@ __device__ __forceinline__ void attn_prefill_g4(const GhAttnArgs& a) {
     // the grid takes L = k, workgroup k + T/2 takes L = T - 1 - k: with the grid dispatched
     // round-robin over the CUs and two workgroups resident per CU, the pair that shares a CU
     // carries one heavy and one light causal block instead of two equal ones.
-    const uint32_t T = nqb * a.kv_heads, k = blockIdx.x + nqb * blockIdx.y, half = (T + 1) / 2;
-    const uint32_t L = k < half ? k : T - 1 - (k - half);  // grid: (nqb, kv_heads)
-    const uint32_t qb = nqb - 1 - L / a.kv_heads, kvh = L % a.kv_heads, h = kvh * 4 + wave;
-    const uint32_t q0 = qb * kPQ;
+    const uint32_t ng = a.q_heads / HW;  // head groups
+    const uint32_t T = nqb * ng, k = blockIdx.x + nqb * blockIdx.y, half = (T + 1) / 2;
+    const uint32_t L = k < half ? k : T - 1 - (k - half);  // grid: (nqb, ng, splits)
+    const uint32_t qb = nqb - 1 - L / ng, hg = L % ng, kvh = hg * HW / G, h = hg * HW + wave % HW;
+    const uint32_t q0 = qb * kPQ, qw = q0 + 16 * QT * (wave / HW);  // the block's, this wave's first row
     const uint32_t kv_end = a.base + min(q0 + kPQ, a.rows);  // keys 0 .. kv_end-1 are visible
-    const uint32_t ntiles = (kv_end + kPK - 1) / kPK;
+    uint32_t tile0 = 0, ntiles = (kv_end + kPK - 1) / kPK;
+    if constexpr (SPLIT) {
+        const uint32_t per = (attn_tiles(a, nqb - 1, kPQ) + a.splits - 1) / a.splits;
+        tile0 = blockIdx.z * per;
+        ntiles = min(tile0 + per, ntiles);
+        if (tile0 >= ntiles) return;  // workgroup-uniform; gh_attn_merge reads no partial of such a split
+    }
     const size_t kv_row = (size_t)a.kv_heads * 128;
     const size_t cache0 = (size_t)a.layer * a.context * kv_row + (size_t)kvh * 128;
     const uint16_t* kc = (const uint16_t*)a.kc + cache0;
@@ -712,14 +733,14 @@ __device__ __forceinline__ void attn_prefill_g4(const GhAttnArgs& a) {
     ah8 qf[QT][4];
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
-        const uint32_t r = min(q0 + 16 * t + fr, a.rows - 1);
+        const uint32_t r = min(qw + 16 * t + fr, a.rows - 1);
         const GH_GLOBAL uint4* qp = gh_gp<uint4>(a.q + (((uint64_t)r * a.q_heads + h) * 128 + 8 * fg) * 2);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) qf[t][ks] = __builtin_bit_cast(ah8, qp[4 * ks]);
     }
     uint32_t qpos[QT];
 #pragma unroll
-    for (int t = 0; t < QT; ++t) qpos[t] = a.base + q0 + 16 * t + fr;
+    for (int t = 0; t < QT; ++t) qpos[t] = a.base + qw + 16 * t + fr;
 
     af4 o[8][QT];
     float m[QT], l[QT];
@@ -732,7 +753,7 @@ __device__ __forceinline__ void attn_prefill_g4(const GhAttnArgs& a) {
     }
 
     const uint32_t kv_row32 = (uint32_t)kv_row;
-    kv_dma(kc, vc, kv_row32, 0, kv_end, kt[0], vt[0]);
+    kv_dma(kc, vc, kv_row32, tile0 * kPK, kv_end, kt[0], vt[0]);
     // the query fragments are taken here, so the compiler settles their loads before the tile
     // loop (it does not see the explicit wait below) and puts no load wait inside the loop
 #pragma unroll
@@ -746,7 +767,7 @@ __device__ __forceinline__ void attn_prefill_g4(const GhAttnArgs& a) {
     const uint32_t first_pos = a.base + q0;
     auto step = [&](uint32_t tile, auto masked) {
         constexpr bool kMask = decltype(masked)::value;
-        const uint32_t cur = tile & 1u, t0 = tile * kPK;
+        const uint32_t cur = (tile - tile0) & 1u, t0 = tile * kPK;
         const bool more = tile + 1 < ntiles;
         // the next tile goes into the other buffers, whose reads ended before the last barrier
         if (more) kv_dma(kc, vc, kv_row32, t0 + kPK, kv_end, kt[cur ^ 1u], vt[cur ^ 1u]);
@@ -781,12 +802,17 @@ __device__ __forceinline__ void attn_prefill_g4(const GhAttnArgs& a) {
                         if (t0 + 16 * kk + 4 * fg + e > qpos[t]) v[kk][e] = -__builtin_inff();
                     mx = fmaxf(mx, v[kk][e]);
                 }
-            // sl2 > 0, so the row max of the scaled scores is sl2 · (row max of the raw ones);
-            // finite: key 0 is in tile 0. v_exp_f32 directly: weights below 2^-126 (flushed
-            // to zero) are far below the FP32 accumulation error of the sums they enter.
-            const float m_new = fmaxf(m[t], xor_max(mx) * sl2);
-            const float f = __builtin_amdgcn_exp2f(m[t] - m_new);
+            // sl2 > 0, so the row max of the scaled scores is sl2 · (row max of the raw ones).
+            // v_exp_f32 directly: weights below 2^-126 (flushed to zero) are far below the
+            // FP32 accumulation error of the sums they enter. Until a row has seen a key of
+            // its split (only in masked tiles: a later split's first tile may lie past the row)
+            // m is -inf, and the exponents are taken from 0 so that every weight and the
+            // rescale come out as 0, not NaN.
+            float m_new = fmaxf(m[t], xor_max(mx) * sl2);
+            const float m_old = m[t];
             m[t] = m_new;
+            if constexpr (SPLIT && kMask) m_new = m_new == -__builtin_inff() ? 0.0f : m_new;
+            const float f = __builtin_amdgcn_exp2f(m_old - m_new);
             float sum = 0.0f;
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk)
@@ -827,15 +853,27 @@ __device__ __forceinline__ void attn_prefill_g4(const GhAttnArgs& a) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's DMA of the next tile has landed
         __syncthreads();  // every wave's has, and every read of this tile is done
     };
-    uint32_t tile = 0;
+    uint32_t tile = tile0;
     for (; tile < ntiles && tile * kPK + kPK - 1 <= first_pos; ++tile) step(tile, Flag<false>{});
     for (; tile < ntiles; ++tile) step(tile, Flag<true>{});
-    // O^T tile (j, t): lane holds dims 16 j + 4 fg + e of query row q0 + 16 t + fr
+    // O^T tile (j, t): lane holds dims 16 j + 4 fg + e of query row qw + 16 t + fr
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
-        const uint32_t r = q0 + 16 * t + fr;
-        const float inv = 1.0f / xor_sum(l[t]);
+        const uint32_t r = qw + 16 * t + fr;
+        const float lt = xor_sum(l[t]);
         if (r >= a.rows) continue;
+        if constexpr (SPLIT) {
+            const uint64_t pi = ((uint64_t)r * a.q_heads + h) * a.splits + blockIdx.z;
+            if (fg == 0) {
+                gh_gpw<float>(a.part_m)[pi] = m[t];
+                gh_gpw<float>(a.part_l)[pi] = lt;
+            }
+            GH_GLOBAL float* pp = gh_gpw<float>(a.part_acc) + pi * 128 + 4 * fg;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) *(GH_GLOBAL af4*)(pp + 16 * j) = o[j][t];
+            continue;
+        }
+        const float inv = 1.0f / lt;
         GH_GLOBAL uint16_t* op = gh_gpw<uint16_t>(a.out) + ((size_t)r * a.q_heads + h) * 128 + 4 * fg;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -847,7 +885,49 @@ __device__ __forceinline__ void attn_prefill_g4(const GhAttnArgs& a) {
 }
 }  // namespace
 
-GH_KERNEL __launch_bounds__(256) void gh_attn_prefill_g4(GhAttnArgs a) { attn_prefill_g4<2>(a); }
-// 16 query rows per workgroup: twice the workgroups, for row counts whose 32-row blocks leave
-// CUs idle
-GH_KERNEL __launch_bounds__(256) void gh_attn_prefill_g4_r16(GhAttnArgs a) { attn_prefill_g4<1>(a); }
+// 32 query rows per wave where that fills the CUs, 16 (suffix _r16) otherwise, with key splits
+// (suffix _r16_k) where those leave CUs idle
+#define GH_ATTN_PREFILL(G)                                                                              \
+    GH_KERNEL __launch_bounds__(256) void gh_attn_prefill_g##G(GhAttnArgs a) { attn_prefill<2, G, false>(a); } \
+    GH_KERNEL __launch_bounds__(256) void gh_attn_prefill_g##G##_r16(GhAttnArgs a) {                    \
+        attn_prefill<1, G, false>(a);                                                                   \
+    }                                                                                                   \
+    GH_KERNEL __launch_bounds__(256) void gh_attn_prefill_g##G##_r16_k(GhAttnArgs a) { attn_prefill<1, G, true>(a); }
+GH_ATTN_PREFILL(1)
+GH_ATTN_PREFILL(2)
+GH_ATTN_PREFILL(4)
+GH_ATTN_PREFILL(8)
+
+// The key splits' partials of attn_prefill merged: one wave per (row, query head) pair, two
+// value dims per lane, out = Σ_s 2^(m_s - M) acc_s / Σ_s 2^(m_s - M) l_s with M = max m_s (base-2
+// units), summed in split order. a.pad: rows per query block of the attention launch (its splits
+// past the block's tiles hold no partial). Split 0 holds key 0, so M is finite.
+GH_KERNEL __launch_bounds__(256) void gh_attn_merge(GhAttnArgs a) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t pair = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (pair >= a.rows * a.q_heads) return;  // wave-uniform
+    const uint32_t qb = pair / a.q_heads / a.pad, nqb = (a.rows + a.pad - 1) / a.pad;
+    const uint32_t per = (attn_tiles(a, nqb - 1, a.pad) + a.splits - 1) / a.splits;
+    const uint32_t ns = (attn_tiles(a, qb, a.pad) + per - 1) / per;  // 1 .. splits <= 32
+    const uint64_t p0 = (uint64_t)pair * a.splits;
+    const uint32_t sl = min(lane, ns - 1);
+    const float ms = gh_gp<float>(a.part_m)[p0 + sl], ls = gh_gp<float>(a.part_l)[p0 + sl];
+    const float M = gh_wave_max(ms);
+    const float e = lane < ns ? __builtin_amdgcn_exp2f(ms - M) : 0.0f;
+    const float w = e / gh_wave_sum(e * ls);  // the split's share, as attn_finish weighs them
+    float2 o = make_float2(0.0f, 0.0f);
+    const GH_GLOBAL float2* pa = gh_gp<float2>(a.part_acc) + p0 * 64 + lane;
+    for (uint32_t s0 = 0; s0 < ns; s0 += 8) {
+        float2 p[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) p[i] = pa[(uint64_t)min(s0 + i, ns - 1) * 64];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) {
+            const float ws = s0 + i < ns ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s0 + i)) : 0.0f;
+            o.x += ws * p[i].x;
+            o.y += ws * p[i].y;
+        }
+    }
+    gh_gpw<uint32_t>(a.out)[(uint64_t)pair * 64 + lane] =
+        (uint32_t)gh_f2h(o.x) | ((uint32_t)gh_f2h(o.y) << 16);
+}

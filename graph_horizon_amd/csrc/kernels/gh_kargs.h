@@ -209,8 +209,10 @@ struct GhAttnArgs {
     uint32_t context;
     uint32_t base;
     uint32_t rows;
-    uint32_t splits;   // grid.x: workgroups per (row, kv head), <= 32
+    uint32_t splits;   // decode: workgroups per (row, kv head); prefill: key splits; <= 32
     float scale;
+    uint32_t pad;      // gh_attn_merge: rows per query block
+    uint32_t pad2;
 };
 
 // Device top-k (read_topk): gh_topk_partial keeps the `width` smallest keys of each stripe of

@@ -1,4 +1,4 @@
-"""Prefill attention on the matrix cores (gh_attention_prefill with n >= 32 rows, G = 4)
+"""Prefill attention on the matrix cores (gh_attention_prefill with several rows, every GQA group)
 against the oracle, and against the reference's own prefill-attention test vectors.
 
 Bars:
@@ -78,6 +78,36 @@ def test_prefill_attention_c4_2048(hip):
         want = O.f32(O.attention_decode(q[r * qh * 128:(r + 1) * qh * 128], kc, vc, 128, kvh, qh,
                                         r, 0, ctx))
         _close(got[r], want, f"row {r}")
+    _free(hip, qb, ob, kv.k, kv.v)
+
+
+@pytest.mark.parametrize("qh,kvh", [(8, 8), (16, 8), (32, 8), (64, 8), (12, 3), (24, 3)],
+                         ids=["g1", "g2", "g4", "g8", "g4-kv3", "g8-kv3"])
+@pytest.mark.parametrize("base,n", [(0, 2), (0, 17), (63, 16), (64, 65), (1000, 5), (700, 33), (1, 130),
+                                    (40, 600)])
+def test_prefill_attention_groups_rows_and_key_splits(hip, qh, kvh, base, n):
+    """Every GQA group, at the edges of the 16- and 32-row query blocks and of the 64-key tiles,
+    with the backend's key splits and forced ones: later splits start past some rows' last key
+    (their partials weigh 0), or hold no tile of the block at all."""
+    if n == 600 and qh == 8:
+        n = 2050  # 32-row query tiles for the groups that fill the CUs with them
+    rng = np.random.default_rng(qh * 1000 + kvh + base + n)
+    ctx = base + n + 3
+    kc = O.f16(rng.standard_normal(2 * ctx * kvh * 128).astype(np.float32))
+    vc = O.f16(rng.standard_normal(2 * ctx * kvh * 128).astype(np.float32))
+    q = O.f16(rng.standard_normal(n * qh * 128).astype(np.float32))
+    kv = _kv(hip, 2, ctx, kvh, kc, vc)
+    qb, ob = hip.from_host(q), hip.alloc_buffer(n * qh * 128 * 2)
+    want = O.f32(O.attention_prefill(q, kc, vc, 128, kvh, qh, base, n, 1, ctx))
+    try:
+        for splits in (0, 1, 3, 32):
+            hip.set_attention_splits(splits)
+            hip.attention_prefill(ob, qb, kv, qh, base, n, 1)
+            got = O.f32(hip.download(ob, np.uint16, n * qh * 128))
+            assert np.isfinite(got).all()
+            _close(got, want, f"splits {splits}")
+    finally:
+        hip.set_attention_splits(0)
     _free(hip, qb, ob, kv.k, kv.v)
 
 
