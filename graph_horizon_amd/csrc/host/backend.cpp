@@ -75,9 +75,17 @@ const KernelName kKernels[] = {
     {K_GEMM3_SWIGLU_R96_T128, "gh_gemm3_swiglu_r96_t128"}, {K_GEMM3_SWIGLU_R128_T128, "gh_gemm3_swiglu_r128_t128"},
     {K_GEMM3_SWIGLU_R96, "gh_gemm3_swiglu_r96"},           {K_GEMM4W_SWIGLU_R96, "gh_gemm4w_swiglu_r96"},
     {K_GEMM3_SWIGLU_R128, "gh_gemm3_swiglu_r128"},         {K_GEMM4W_SWIGLU_R128, "gh_gemm4w_swiglu_r128"},
+    {K_GEMM_FEW_Q4K_T8, "gh_gemm_few_q4k_t8"}, {K_GEMM_FEW_Q6K_T8, "gh_gemm_few_q6k_t8"},
+    {K_GEMM_FEW_MIXED_T8, "gh_gemm_few_mixed_t8"},
+    {K_GEMM_FEW_Q4K_T16, "gh_gemm_few_q4k_t16"}, {K_GEMM_FEW_Q6K_T16, "gh_gemm_few_q6k_t16"},
+    {K_GEMM_FEW_MIXED_T16, "gh_gemm_few_mixed_t16"},
+    {K_GEMM_FEW_Q4K_T32, "gh_gemm_few_q4k_t32"}, {K_GEMM_FEW_Q6K_T32, "gh_gemm_few_q6k_t32"},
+    {K_GEMM_FEW_MIXED_T32, "gh_gemm_few_mixed_t32"},
+    {K_GEMM_FEW_Q4K_T48, "gh_gemm_few_q4k_t48"}, {K_GEMM_FEW_Q6K_T48, "gh_gemm_few_q6k_t48"},
+    {K_GEMM_FEW_MIXED_T48, "gh_gemm_few_mixed_t48"},
 };
 
-const char* kModules[] = {"gh_quant", "gh_gemv", "gh_glue", "gh_attention", "gh_gemm"};
+const char* kModules[] = {"gh_quant", "gh_gemv", "gh_glue", "gh_attention", "gh_gemm", "gh_gemm_few"};
 
 constexpr uint32_t kArgmaxBlocks = 256;
 // argmax scratch at the front of the workspace: f32[256] values, u32[256] indices, u32 result
@@ -991,10 +999,14 @@ int gh_embed(gh_backend* b, gh_encoder* enc, const gh_buf* x, const gh_buf* w, u
 
 namespace gh {
 
-// Matrix-core GEMM for n >= kGemmMinTokens: the warp-specialized kernels (512-thread
+// Matrix-core GEMM for n >= kGemmMinTokens: up to kGemmFewMax tokens the few-token kernels
+// (gemm_few.hip), above them the warp-specialized kernels (512-thread
 // workgroups of 256 tokens, or 128 below 256 tokens, x 128 or 96 rows), over FP16 weight
 // copies where registered; K splits over the units when the tiles alone would leave CUs idle.
-constexpr uint32_t kGemmMinTokens = 8;
+constexpr uint32_t kGemmMinTokens = 2;
+// 12288 x 4096 at 48 / 64 tokens 25.7 / 33.4 us against 30.9 / 32.0 in the 128-token tiles, 4096 x 12288
+// 33.0 / 36.9 against 34.8 / 35.8
+constexpr uint32_t kGemmFewMax = 48;
 constexpr uint32_t kGemmTailMaxRows = 8192;  // gh_gemm_tail: two 16-value items per thread
 
 // The launch plan of one GEMM: kernel, row and token tiles, and K splits (every split
@@ -1003,7 +1015,34 @@ struct GemmPlan {
     GhKernel k;
     uint32_t tr, tt, splits;
     uint64_t w16;
+    uint32_t shmem = 0;
 };
+
+// The few-token kernels' launch: the Q4_K kernel for n tokens (+ 1: Q6_K, + 2: mixed), K splits and
+// dynamic LDS. Two blocks per split (both in flight from the start), more only past 32 splits, by
+// in_dim alone, so that a matrix's sums do not depend on the launch it is in.
+struct FewPlan {
+    int k;
+    uint32_t splits, shmem;
+};
+static FewPlan plan_few(uint32_t in_dim, uint32_t n) {
+    const uint32_t nb = in_dim / 256;
+    const uint32_t fit = std::max(1u, (72u * 1024 / 2 / n - 16) / 272);
+    uint32_t per = std::min(std::max(2u, ceil_div(nb, 32u)), fit);
+    const uint32_t splits = ceil_div(nb, per);
+    per = ceil_div(nb, splits);
+    const int k = n < 8     ? K_GEMM_FEW_Q4K_T8
+                  : n <= 16 ? K_GEMM_FEW_Q4K_T16
+                  : n <= 32 ? K_GEMM_FEW_Q4K_T32 : K_GEMM_FEW_Q4K_T48;
+    return FewPlan{k, splits, n * ((per * 256 + 8) + (per * 16 + 8)) * 2};
+}
+
+// The few-token kernel over ga.seg[0 .. nseg), `tiles` row tiles of 128 in all.
+static int launch_few(gh_backend* b, const FewPlan& f, const GhGemmArgs& ga, uint32_t tiles) {
+    bool q4 = true, q6 = true;
+    for (uint32_t i = 0; i < ga.nseg; ++i) (ga.seg[i].fmt == GH_FMT_Q4_K ? q6 : q4) = false;
+    return launch(b, (GhKernel)(f.k + (q4 ? 0 : q6 ? 1 : 2)), f.splits, tiles, 1, 256, &ga, f.shmem);
+}
 
 // Threads per workgroup of a prefill GEMM kernel: the dequantizing 256-token tiles and the
 // 128-row 128-token tiles run eight consumer and four producer waves, every other form eight
@@ -1024,6 +1063,10 @@ static uint32_t gemm_block(GhKernel k) {
 
 static GemmPlan plan_gemm(gh_backend* b, const gh_buf* w, uint32_t n) {
     const uint32_t rows = w->rows, units = w->cols / 64;
+    if (n <= kGemmFewMax) {
+        const FewPlan f = plan_few(w->cols, n);
+        return GemmPlan{(GhKernel)(f.k + (w->format == GH_FMT_Q4_K ? 0 : 1)), ceil_div(rows, 128), 1, f.splits, 0, f.shmem};
+    }
     // Batches of 128 tokens or fewer take 128-token tiles (kGemmTallTokens).
     const bool tall = n >= kGemmTallTokens;
     // splits: at most 16, and at least 8 units of 64 k per split (12 in the 128-token tiles,
@@ -1084,6 +1127,11 @@ static int gemm_kernel(gh_backend* b, const GemmPlan& p, uint64_t out, uint64_t 
     ga.splits = p.splits;
     ga.epi = epi;
     ga.aux = aux;
+    if (p.shmem) {  // few tokens: splits fastest
+        ga.nseg = 1;
+        ga.seg[0] = GhGemmSeg{ga.w, out, w->rows, w->format, 0, 0, 0, 0};
+        return launch_few(b, plan_few(w->cols, n), ga, p.tr);
+    }
     return launch(b, p.k, p.tr, p.tt, p.splits, gemm_block(p.k), &ga);
 }
 
@@ -1137,7 +1185,30 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
     const uint64_t cells = (uint64_t)n * wg->rows;
     if (!fits(a, (uint64_t)n * wg->cols * 2) || !fits(out, cells * 2) || !fits(gate, cells * 2))
         return fail(b, GH_E_RANGE, "gemm swiglu: buffer too small");
-    // 8-128 tokens, Q4_K gate and up whose row pairs fill at most one wave of workgroups: one
+    if (n <= kGemmFewMax && wg->rows % 4 == 0) {
+        // few tokens: both matrices in one launch, partials [2][splits][n][rows] for the shared reduce
+        const FewPlan f = plan_few(wg->cols, n);
+        const uint64_t half = (uint64_t)f.splits * cells;
+        int rc = ensure_workspace(b, 2 * half * 4);
+        if (rc) return rc;
+        GhGemmArgs ga{};
+        ga.x = a->addr;
+        ga.part = (uint64_t)((char*)b->ws + kArgmaxBytes);
+        ga.in_dim = wg->cols;
+        ga.rows = wg->rows;
+        ga.n = n;
+        ga.splits = f.splits;
+        ga.nseg = 2;
+        const uint32_t tiles = ceil_div(wg->rows, 128);
+        ga.seg[0] = GhGemmSeg{wg->addr, 0, wg->rows, wg->format, 0, 0, 0, 0};
+        ga.seg[1] = GhGemmSeg{wu->addr, 0, wg->rows, wu->format, tiles, 0, 0, (uint32_t)half};
+        rc = launch_few(b, f, ga, 2 * tiles);
+        if (rc) return rc;
+        ga.out = out->addr;
+        return launch(b, K_GEMM_REDUCE_SWIGLU, (uint32_t)std::min<uint64_t>(ceil_div(cells / 4, (uint64_t)256), 4096),
+                      1, 1, 256, &ga);
+    }
+    // 49-128 tokens, Q4_K gate and up whose row pairs fill at most one wave of workgroups: one
     // launch of 96-row tiles (48 gate rows + the same 48 up rows) or, where those would be more
     // than the CUs, 128-row tiles (64 + 64, eight consumers), K unsplit, silu_mul in the
     // epilogue — no FP32 partials or split reduce (8B 128 x 4096 -> 2 x 12288: 256 tiles of
@@ -1249,7 +1320,7 @@ bool gemm_multi_applies(uint32_t n) { return n >= kGemmMinTokens; }
 int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint32_t nseg, uint32_t n,
                   const GhRopeTable* rope, uint32_t base, uint32_t head_dim) {
     constexpr uint32_t BR = 128;
-    if (nseg == 0 || nseg > 3 || !gemm_multi_applies(n)) return fail(b, GH_E_UNSUPPORTED, "gemm multi: 1..3 matrices, n >= 8");
+    if (nseg == 0 || nseg > 3 || !gemm_multi_applies(n)) return fail(b, GH_E_UNSUPPORTED, "gemm multi: 1..3 matrices, n >= 2");
     const uint32_t in_dim = segs[0].w->cols;
     GhGemmArgs ga{};
     uint32_t tiles = 0, total = 0;
@@ -1274,7 +1345,9 @@ int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint3
     const bool tall = n >= kGemmTallTokens;
     bool copies = tall;
     for (uint32_t i = 0; i < nseg; ++i) copies = copies && b->w16.count(segs[i].w->addr);
-    const uint32_t tt = ceil_div(n, tall ? 256u : 128u), units = in_dim / 64;
+    const bool few = n <= kGemmFewMax;
+    const FewPlan fp = few ? plan_few(in_dim, n) : FewPlan{};
+    const uint32_t tt = few ? 1 : ceil_div(n, tall ? 256u : 128u), units = in_dim / 64;
     // splits: the CUs over the tiles, at most 16 and at least 8 units per split (12 in the
     // 128-token tiles, as op_gemm), none empty
     const uint32_t min_units = tall ? 8u : 12u;
@@ -1285,6 +1358,7 @@ int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint3
         if (s == splits) break;
         splits = s;
     }
+    if (few) splits = fp.splits;
     if (copies)
         for (uint32_t i = 0; i < nseg; ++i) ga.seg[i].w = b->w16.at(segs[i].w->addr);
     ga.x = a->addr;
@@ -1308,7 +1382,7 @@ int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint3
         ga.part = (uint64_t)((char*)b->ws + kArgmaxBytes);
     }
     const GhKernel k = copies ? K_GEMM4W_MIXED_R128 : tall ? K_GEMM3_MIXED_R128 : K_GEMM3_MIXED_R128_T128;
-    int rc = launch(b, k, tiles, tt, splits, gemm_block(k), &ga);
+    int rc = few ? launch_few(b, fp, ga, tiles) : launch(b, k, tiles, tt, splits, gemm_block(k), &ga);
     if (rc) return rc;
     if (splits > 1) {
         const uint64_t npairs = (uint64_t)n * total / 2;
@@ -1349,7 +1423,13 @@ static int gemv_launch(gh_backend* b, const gh_buf* out, const gh_buf* a, const 
     if (w->cols != in_dim || w->rows != out_dim) return fail(b, GH_E_INVALID, "matmul: weight shape mismatch");
     if (!fits(a, (uint64_t)n * in_dim * 2) || !fits(out, (uint64_t)n * out_dim * (f32 ? 4 : 2)))
         return fail(b, GH_E_RANGE, "matmul: buffer too small");
-    if (!f32 && n >= kGemmMinTokens) return op_gemm(b, out->addr, a, w, n);
+    if (in_dim / 64 > 256 && n < 8) return fail(b, GH_E_UNSUPPORTED, "gemv: in_dim above 16384");
+    // Fewer than 8 tokens of a small matrix: the GEMV reads it once per token, mostly from the caches,
+    // without the GEMM's split reduce (about 2.5 us + 0.3 us per MB and token against 9.5 + 0.14 per MB:
+    // 4096 x 4096 Q4_K at 2 / 5 tokens 8.3 / 16.1 us against 9.6 / 10.2, 1024 x 4096 Q6_K 4.9 / 8.6
+    // against 10.0 / 10.5, 12288 x 4096 14.9 / 32.7 against 13.3 / 13.4)
+    const bool small = n < 8 && n * w->bytes <= (uint64_t)24 << 20;
+    if (!f32 && n >= kGemmMinTokens && !small) return op_gemm(b, out->addr, a, w, n);
     GemvSeg seg{w, out->addr, f32 ? (uint32_t)GH_EPI_F32 : (uint32_t)GH_EPI_F16};
     return op_gemv(b, &seg, 1, a, n, 0, nullptr, 0, nullptr);
 }

@@ -113,6 +113,19 @@ enum GhKernel : int {
     K_GEMM4W_SWIGLU_R96,
     K_GEMM3_SWIGLU_R128,
     K_GEMM4W_SWIGLU_R128,
+    // few tokens: Q4_K, Q6_K and mixed by most tokens (fewer than 8, 16, 32, 48)
+    K_GEMM_FEW_Q4K_T8,
+    K_GEMM_FEW_Q6K_T8,
+    K_GEMM_FEW_MIXED_T8,
+    K_GEMM_FEW_Q4K_T16,
+    K_GEMM_FEW_Q6K_T16,
+    K_GEMM_FEW_MIXED_T16,
+    K_GEMM_FEW_Q4K_T32,
+    K_GEMM_FEW_Q6K_T32,
+    K_GEMM_FEW_MIXED_T32,
+    K_GEMM_FEW_Q4K_T48,
+    K_GEMM_FEW_Q6K_T48,
+    K_GEMM_FEW_MIXED_T48,
     K_COUNT
 };
 
@@ -236,7 +249,7 @@ constexpr uint64_t kMinViewAlignment = 16;
 int op_gemv(gh_backend* b, const GemvSeg* segs, uint32_t nseg, const gh_buf* x, uint32_t n,
             uint32_t base, const void* pos_ptr, uint32_t head_dim, const gh_buf* up,
             const gh_buf* norm = nullptr, float eps = 0.0f, const GhRopeTable* rope = nullptr);
-// Epilogue of a prefill GEMM (n >= 8 tokens). epi/aux: GH_GEMM_EPI_SILU with the FP16 gate
+// Epilogue of a prefill GEMM (n >= 2 tokens). epi/aux: GH_GEMM_EPI_SILU with the FP16 gate
 // (out = silu_mul(gate, f16(acc))). resid != 0: the output row is folded into the FP32 residual
 // x[n][out_dim] (residual_add) and, with norm != 0, its RMSNorm written to normed — the bits of
 // the separate reduce, residual_add and rmsnorm_x ops (out then only holds the FP16 projection).
@@ -251,7 +264,7 @@ struct GemmEpi {
 int op_gemm(gh_backend* b, uint64_t out, const gh_buf* a, const gh_buf* w, uint32_t n,
             const GemmEpi* e = nullptr);
 bool gemm_epi_applies(uint32_t n, uint32_t out_dim, bool tail);
-// SwiGLU's gate and up projections of one FP16 input (n >= 8 tokens) and silu_mul, with one
+// SwiGLU's gate and up projections of one FP16 input (n >= 2 tokens) and silu_mul, with one
 // split reduce for both GEMMs where they split K; `gate` receives the gate's FP16 output only
 // where they do not. The values of op_gemm(gate), op_gemm(up) and silu_mul.
 int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const gh_buf* a, const gh_buf* wg,
@@ -267,7 +280,7 @@ bool gemm_rope_applies(uint32_t n, uint32_t out_dim, uint32_t head_dim, const Gh
 // the dequantizing kernels exactly, where a copy's four-fold weight stream costs more. Both
 // forms of a batch size share one tile and split plan, so they give the same bits.
 constexpr uint32_t kGemmTallTokens = 129;
-// Several projections of one FP16 input (n >= 8 tokens) in one warp-specialized launch (row
+// Several projections of one FP16 input (n >= 2 tokens) in one warp-specialized launch (row
 // tiles of 128, each in its matrix's format) and one split reduce that writes each matrix's
 // FP16 output and applies its RoPE role (GH_GEMM_ROLE_*; rows of head_dim, positions base + t)
 // — the values of separate gh_matmul_batched launches and op_rope.
@@ -280,7 +293,7 @@ bool gemm_multi_applies(uint32_t n);
 int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint32_t nseg, uint32_t n,
                   const GhRopeTable* rope, uint32_t base, uint32_t head_dim);
 // gh_matmul_batched then op_rope(role, positions base + t) on its output, the rotation folded
-// into the split reduce when the GEMM splits K (n >= 8 tokens, out_dim a multiple of head_dim).
+// into the split reduce when the GEMM splits K (n >= 2 tokens, out_dim a multiple of head_dim).
 size_t attention_workspace(uint32_t rows, uint32_t q_heads, uint32_t splits);
 uint32_t attention_splits(const gh_backend* b, uint32_t max_len, uint32_t kv_heads, uint32_t rows);
 int ensure_counters(gh_backend* b, size_t slots);

@@ -258,7 +258,7 @@ int layer(gh_model* m, gh_encoder* enc, const Scratch& s, uint32_t li, uint32_t 
                                         {&w[GH_T_ATTN_V], &vd, GH_GEMM_ROLE_PLAIN}};
             if (!rc) rc = op_gemm_multi(b, &s.normed, qkv, 3, rows, &m->rope, base, c.key_length);
         } else {
-            // chunks of fewer than 8 rows (the GEMV): rope_yarn_batched (prefill/layer.rs:79-89)
+            // one row of a model whose decode is not fused (the GEMV): rope_yarn_batched (prefill/layer.rs:79-89)
             // on the Q rows and, in place, on the K cache rows
             if (!rc) rc = gh_matmul_batched(b, enc, &s.q, &s.normed, &w[GH_T_ATTN_Q], d, qw, rows);
             if (!rc) rc = gh_matmul_batched(b, enc, &kd, &s.normed, &w[GH_T_ATTN_K], d, kw, rows);

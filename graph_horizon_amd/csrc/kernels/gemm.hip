@@ -148,79 +148,11 @@ __device__ __forceinline__ void load_wblock(const GhGemmArgs& a, uint32_t r0, ui
 template <uint32_t FMT, int BR>
 __device__ __forceinline__ void store_w(uint32_t u, const WStage& ws, _Float16* wb,
                                         uint32_t tid = threadIdx.x) {
-#pragma clang fp contract(off)
     const uint32_t row = tid % BR, part = tid / BR;
     _Float16* dst = wb + row * LDK;
-    const uint32_t qw[4] = {ws.q.x, ws.q.y, ws.q.z, ws.q.w};
     uint32_t lo[8], hi[8];
-    if constexpr (FMT == kQ4K) {
-        const uint32_t g = u & 3u;
-        uint32_t sc0, mn0, sc1, mn1;
-        gh_q4k_scale_min(ws.hd, 2 * g, sc0, mn0);
-        gh_q4k_scale_min(ws.hd, 2 * g + 1, sc1, mn1);
-        const float d = gh_h2f(ws.hd.x & 0xFFFFu), dmin = gh_h2f(ws.hd.x >> 16);
-        const float d1 = d * (float)sc0, m1 = dmin * (float)mn0;
-        const float d2 = d * (float)sc1, m2 = dmin * (float)mn1;
-        // nibbles four at a time: byte e of lo4 / hi4 is the low / high nibble of byte e.
-        // d·sc and dmin·mn are exact in FP32 (an FP16 times a 6-bit integer), and so is
-        // (d·sc)·q for a 4-bit q (at most 21 significant bits): the reference's product,
-        // then difference, rounds once, as one FMA does, so the FMA gives the same FP32 value.
-        auto w2 = [](uint32_t q4, int e, float sc, float mn) __attribute__((always_inline)) {
-            typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
-            const float f0 = (float)((q4 >> (8 * e)) & 0xFFu), f1 = (float)((q4 >> (8 * e + 8)) & 0xFFu);
-            float v0 = __builtin_fmaf(sc, f0, -mn), v1 = __builtin_fmaf(sc, f1, -mn);
-            // the FP32 values are rounded to FP16 as a second step (v_cvt_pk_f16_f32), not fused
-            // into one rounding of the exact value (v_fma_mix), which differs on FP16 ties
-            asm volatile("" : "+v"(v0), "+v"(v1));
-            const hv2 r = {(_Float16)v0, (_Float16)v1};
-            return __builtin_bit_cast(uint32_t, r);
-        };
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint32_t lo4 = qw[j] & 0x0F0F0F0Fu, hi4 = (qw[j] >> 4) & 0x0F0F0F0Fu;
-            // opaque: with the masks' known zero bits the compiler would extract each byte
-            // separately instead of converting it in place (v_cvt_f32_ubyte1..3)
-            asm volatile("" : "+v"(lo4), "+v"(hi4));
-            lo[2 * j] = w2(lo4, 0, d1, m1);
-            lo[2 * j + 1] = w2(lo4, 2, d1, m1);
-            hi[2 * j] = w2(hi4, 0, d2, m2);
-            hi[2 * j + 1] = w2(hi4, 2, d2, m2);
-        }
-    } else {
-        // part 0: ql plane a -> quarters 0 (low nibble, qh bits 0-1) and 2 (high, bits 4-5);
-        // part 1: plane b -> quarters 1 (bits 2-3) and 3 (bits 6-7). Scale of quarter q:
-        // int8 scales[8s + h + 2q]. Four quants per dword: the nibble and the two high bits
-        // are combined byte-parallel into unsigned 6-bit values u, and each weight is
-        // (u - 32)·da = u·da + (-32·da) (the bias exact: a power-of-two multiple), one fused
-        // multiply-add rounded once to FP16.
-        const uint32_t s = (u >> 1) & 1u, h = u & 1u;
-        const uint32_t scw[4] = {ws.hd.x, ws.hd.y, ws.hd.z, ws.hd.w};
-        const uint32_t ia = 8 * s + h + 2 * part, ib = ia + 4;
-        const float d = gh_h2f(ws.d);
-        const float da = d * (float)(int8_t)(scw[ia >> 2] >> (8 * (ia & 3u)));
-        const float db = d * (float)(int8_t)(scw[ib >> 2] >> (8 * (ib & 3u)));
-        const float na = -32.0f * da, nb = -32.0f * db;
-        const uint32_t qh[4] = {ws.qh.x, ws.qh.y, ws.qh.z, ws.qh.w};
-        // the two high bits of each quant moved to bits 4-5 of its byte in one shift:
-        // ((qh >> 2 part) & 3) << 4 = (qh << (4 - 2 part)) & 0x30, ((qh >> (4 + 2 part)) & 3) << 4
-        // = (qh >> 2 part) & 0x30 (part is 0 or 1)
-        const uint32_t sl = 4 - 2 * part, sh = 2 * part;
-        auto w2 = [](uint32_t q4, int e, float sc, float bias) __attribute__((always_inline)) {
-            typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
-            const float f0 = (float)((q4 >> (8 * e)) & 0xFFu), f1 = (float)((q4 >> (8 * e + 8)) & 0xFFu);
-            const hv2 r = {(_Float16)__builtin_fmaf(f0, sc, bias), (_Float16)__builtin_fmaf(f1, sc, bias)};
-            return __builtin_bit_cast(uint32_t, r);
-        };
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t qa4 = (qw[j] & 0x0F0F0F0Fu) | ((qh[j] << sl) & 0x30303030u);
-            const uint32_t qb4 = ((qw[j] >> 4) & 0x0F0F0F0Fu) | ((qh[j] >> sh) & 0x30303030u);
-            lo[2 * j] = w2(qa4, 0, da, na);
-            lo[2 * j + 1] = w2(qa4, 2, da, na);
-            hi[2 * j] = w2(qb4, 0, db, nb);
-            hi[2 * j + 1] = w2(qb4, 2, db, nb);
-        }
-    }
+    if constexpr (FMT == kQ4K) gh_w16_q4k(ws.q, ws.hd, u & 3u, lo, hi);
+    else gh_w16_q6k(ws.q, ws.qh, ws.hd, ws.d, (u >> 1) & 1u, u & 1u, part, lo, hi);
     // low nibbles (quarter 2·part for Q6_K): positions 16·part + i; high: 32 + 16·part + i
     *(uint4*)(dst + 16 * part) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
     *(uint4*)(dst + 16 * part + 8) = make_uint4(lo[4], lo[5], lo[6], lo[7]);
@@ -818,6 +750,27 @@ GH_KERNEL __launch_bounds__(512) void gh_gemm4w_mixed_r128(GhGemmArgs a) {
         gemm4_body<kQ6K, 128>(m, lds, bx, blockIdx.y, blockIdx.z, a.rows, a.seg[s].col0);
 }
 
+// add(load(k)) for the splits k = 0 .. splits - 1 in order, up to 8 partials requested before any is
+// summed (clamped indices past the last, no branch around the loads): summed one load at a time, every
+// split waits out a round trip.
+template <uint32_t B, class L, class A>
+__device__ __forceinline__ void sum_batches(uint32_t splits, const L& load, const A& add) {
+    for (uint32_t k0 = 0; k0 < splits; k0 += B) {
+        decltype(load(0u)) p[B];
+#pragma unroll
+        for (uint32_t k = 0; k < B; ++k) p[k] = load(min(k0 + k, splits - 1));
+#pragma unroll
+        for (uint32_t k = 0; k < B; ++k)
+            if (k0 + k < splits) add(p[k]);
+    }
+}
+template <class L, class A>
+__device__ __forceinline__ void sum_splits(uint32_t splits, const L& load, const A& add) {
+    if (splits <= 2) sum_batches<2>(splits, load, add);
+    else if (splits <= 4) sum_batches<4>(splits, load, add);
+    else sum_batches<8>(splits, load, add);
+}
+
 // Sum split-K partials in split order, round to FP16: out[i] = f16(Σ_s part[s][i]).
 GH_KERNEL __launch_bounds__(256) void gh_gemm_reduce(GhGemmArgs a) {
     const uint64_t total = (uint64_t)a.n * a.rows;
@@ -825,7 +778,8 @@ GH_KERNEL __launch_bounds__(256) void gh_gemm_reduce(GhGemmArgs a) {
     const uint64_t groups = min((total + 255) / 256, (uint64_t)4096);
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += groups * 256) {
         float s = 0.0f;
-        for (uint32_t k = 0; k < a.splits; ++k) s += gh_gp<float>(a.part)[k * total + i];
+        sum_splits(
+            a.splits, [&](uint32_t k) { return gh_gp<float>(a.part)[k * total + i]; }, [&](float p) { s += p; });
         gemm_store(a, i, s);
     }
 }
@@ -842,17 +796,21 @@ GH_KERNEL __launch_bounds__(256) void gh_gemm_reduce_swiglu(GhGemmArgs a) {
     const GH_GLOBAL float4* p = gh_gp<float4>(a.part);
     for (uint64_t q = (uint64_t)blockIdx.x * 256 + threadIdx.x; q < nq; q += groups * 256) {
         float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f), u = g;
-        for (uint32_t z = 0; z < a.splits; ++z) {
-            const float4 pg = p[z * nq + q], pu = p[(a.splits + z) * nq + q];
-            g.x += pg.x;
-            g.y += pg.y;
-            g.z += pg.z;
-            g.w += pg.w;
-            u.x += pu.x;
-            u.y += pu.y;
-            u.z += pu.z;
-            u.w += pu.w;
-        }
+        struct GU {
+            float4 g, u;
+        };
+        sum_splits(
+            a.splits, [&](uint32_t z) { return GU{p[z * nq + q], p[(a.splits + z) * nq + q]}; },
+            [&](const GU& v) {
+                g.x += v.g.x;
+                g.y += v.g.y;
+                g.z += v.g.z;
+                g.w += v.g.w;
+                u.x += v.u.x;
+                u.y += v.u.y;
+                u.z += v.u.z;
+                u.w += v.u.w;
+            });
         const uint32_t o0 = gh_silu_mul_h(gh_f2h(g.x), gh_f2h(u.x)) | ((uint32_t)gh_silu_mul_h(gh_f2h(g.y), gh_f2h(u.y)) << 16);
         const uint32_t o1 = gh_silu_mul_h(gh_f2h(g.z), gh_f2h(u.z)) | ((uint32_t)gh_silu_mul_h(gh_f2h(g.w), gh_f2h(u.w)) << 16);
         gh_gpw<uint2>(a.out)[q] = make_uint2(o0, o1);
@@ -871,11 +829,12 @@ GH_KERNEL __launch_bounds__(256) void gh_gemm_reduce_seg(GhGemmArgs a) {
     for (uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < npairs; k += groups * 256) {
         const uint64_t i = 2 * k;
         float s0 = 0.0f, s1 = 0.0f;
-        for (uint32_t z = 0; z < a.splits; ++z) {
-            const float2 p = gh_gp<float2>(a.part)[(z * total + i) / 2];
-            s0 += p.x;
-            s1 += p.y;
-        }
+        sum_splits(
+            a.splits, [&](uint32_t z) -> float2 { return gh_gp<float2>(a.part)[(z * total + i) / 2]; },
+            [&](const float2& p) {
+                s0 += p.x;
+                s1 += p.y;
+            });
         const uint32_t t = (uint32_t)(i / a.rows), col = (uint32_t)(i % a.rows);
         uint32_t sg = 0;
         for (uint32_t j = 1; j < a.nseg; ++j)
@@ -913,7 +872,7 @@ GH_KERNEL __launch_bounds__(1024) void gh_gemm_tail(GhGemmArgs a) {
     __shared__ float red[4];
     __shared__ float4 ys[2048];  // the updated residual row (rows <= 8192)
     // Pass 1, coalesced: thread t takes float4 j0 + t (a wave's loads cover whole lines), 1024
-    // per round. Every load of a round and a group of four splits is requested before any is
+    // per round. Every load of a round and a group of splits (sum_splits) is requested before any is
     // summed (clamped indices, no branch around the loads); the splits are summed in order, the
     // sum rounded to FP16, added into the residual, and the new row kept in LDS.
     for (uint32_t j0 = 0; j0 < n4; j0 += 1024) {  // launch-uniform: one round up to 4096 rows
@@ -921,20 +880,14 @@ GH_KERNEL __launch_bounds__(1024) void gh_gemm_tail(GhGemmArgs a) {
         float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         const float4 xv = x[c];
         if (a.splits > 1) {
-            for (uint32_t k0 = 0; k0 < a.splits; k0 += 4) {
-                float4 p[4];
-#pragma unroll
-                for (uint32_t kk = 0; kk < 4; ++kk)
-                    p[kk] = gh_gp<float4>(a.part)[(min(k0 + kk, a.splits - 1) * total + row0) / 4 + c];
-#pragma unroll
-                for (uint32_t kk = 0; kk < 4; ++kk)
-                    if (k0 + kk < a.splits) {
-                        s.x += p[kk].x;
-                        s.y += p[kk].y;
-                        s.z += p[kk].z;
-                        s.w += p[kk].w;
-                    }
-            }
+            sum_splits(
+                a.splits, [&](uint32_t k) -> float4 { return gh_gp<float4>(a.part)[(k * total + row0) / 4 + c]; },
+                [&](const float4& p) {
+                    s.x += p.x;
+                    s.y += p.y;
+                    s.z += p.z;
+                    s.w += p.w;
+                });
         } else {
             const uint2 o = gh_gp<uint2>(a.out)[row0 / 4 + c];
             s = make_float4(gh_h2f(o.x & 0xFFFFu), gh_h2f(o.x >> 16), gh_h2f(o.y & 0xFFFFu), gh_h2f(o.y >> 16));

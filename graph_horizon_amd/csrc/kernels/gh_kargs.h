@@ -110,7 +110,7 @@ struct GhGemmSeg {
     uint32_t tile0;
     uint32_t col0;
     uint32_t role;   // split reduce: GH_GEMM_ROLE_*
-    uint32_t pad;
+    uint32_t part0;  // gh_gemm_few_mixed_*: its partials start at this float of `part`
 };
 
 // Prefill GEMM (gemm.hip): out f16 [n][rows] (or FP32 split partials [splits][n][rows]).

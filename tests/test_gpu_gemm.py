@@ -126,6 +126,54 @@ def test_gemm_equals_gemv_within_tolerance_at_threshold(hip):
         hip.free_buffer(b)
 
 
+@pytest.mark.parametrize("fmt", [F.FMT_Q4_K, F.FMT_Q6_K], ids=["q4k", "q6k"])
+@pytest.mark.parametrize("rows,in_dim,n", [
+    (13000, 4096, 2), (13000, 4096, 5), (16001, 3072, 7),  # exact weights; an odd block count
+    (128, 256, 8), (1, 512, 9), (129, 768, 16), (300, 4096, 17), (1000, 1280, 32), (257, 2048, 33),
+    (96, 16640, 40),  # 65 blocks: three per split, the last split shorter
+    (640, 5120, 48), (640, 5120, 49),
+])
+def test_gemm_few_tokens(hip, fmt, rows, in_dim, n):
+    """The few-token kernels at the edges of their token tiles, row tiles and K splits: below 8
+    tokens against the unrounded weights, from 8 against the FP16-rounded ones."""
+    w, a16, got = _run(hip, fmt, rows, in_dim, n, 31 + rows + n)
+    assert np.isfinite(got).all()
+    _check_fp64(fmt, w, a16, got, rows, in_dim, n, f"{fmt} {rows}x{in_dim} n={n}", f16_weights=n >= 8)
+
+
+@pytest.mark.parametrize("fmt", [F.FMT_Q4_K, F.FMT_Q6_K], ids=["q4k", "q6k"])
+@pytest.mark.parametrize("x_scale", [2.0 ** -20, 2.0 ** -10, 400.0])
+def test_gemm_few_tokens_exact_extremes(hip, fmt, x_scale):
+    """Exact weights at the ends of their formats (scales -128 and 127 and quants 0 and 63 in Q6_K,
+    whose products exceed FP16's integers; scales and minima 63 in Q4_K, where the minima almost
+    cancel the quants) over activations from FP16's subnormals to 1600, against fp64."""
+    rows, in_dim, n = 16384, 4096, 3
+    rng = np.random.default_rng(5)
+    w = synth.quant_blocks(rng, fmt, rows, in_dim, 0.002).reshape(-1, 144 if fmt == F.FMT_Q4_K else 210).copy()
+    if fmt == F.FMT_Q4_K:
+        w[::3, 4:16] = 255
+        w[1::3, 2:4] = (w[1::3, 0:2].view(np.float16) * np.float16(7.5)).view(np.uint8)
+    else:
+        w[::3, 192:208] = 128  # -128
+        w[1::3, 192:208] = 127
+        w[::2, :192] = rng.integers(0, 2, (len(w[::2]), 192)).astype(np.uint8) * 255
+    w = w.reshape(-1)
+    a16 = O.f16((rng.standard_normal(n * in_dim) * x_scale).astype(np.float32))
+    wb, ab, ob = hip.load_weight(fmt, w, in_dim, rows), hip.from_host(a16), hip.alloc_buffer(n * rows * 2)
+    hip.matmul_batched(ob, ab, wb, in_dim, rows, n)
+    got = O.f32(hip.download(ob, np.uint16, n * rows)).reshape(n, rows).astype(np.float64)
+    a = O.f32(a16).astype(np.float64).reshape(n, in_dim)
+    for r0 in range(0, rows, 4096):
+        deq = O.dequant(fmt, w, rows, in_dim)[r0:r0 + 4096].astype(np.float64)
+        want, terms = a @ deq.T, np.abs(a) @ np.abs(deq).T
+        # FP16 output (2^-11 relative, 2^-25 where it is subnormal) and FP32 sums
+        tol = 1e-3 * np.abs(want) + 2e-6 * terms + 2.0 ** -24
+        over = np.abs(want) > 65000
+        assert (np.abs(got[:, r0:r0 + 4096] - want) <= tol)[~over].all(), (fmt, x_scale)
+    for b in (wb, ab, ob):
+        hip.free_buffer(b)
+
+
 def _lcg(count, seed=0x9E3779B9):
     """The reference test generator, seed = seed * 1664525 + 1013904223 (mod 2^32), as the
     array of its first `count` outputs (blocks of M steps advanced with the M-step map)."""
