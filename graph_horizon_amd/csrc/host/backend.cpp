@@ -256,21 +256,34 @@ int ensure_rope(gh_backend* b, GhRopeTable& t, const gh_yarn* y, uint32_t positi
     return GH_OK;
 }
 
-int op_rope(gh_backend* b, const GhRopeTable& t, const gh_buf* x, uint32_t heads,
-            uint32_t head_dim, uint32_t base, uint32_t rows, uint32_t role, const void* pos_ptr) {
+// Query heads `q` (post-scaled) and key heads `k` (either may be null) of `rows` rows in one launch.
+static int rope_launch(gh_backend* b, const GhRopeTable& t, const gh_buf* q, const gh_buf* k, uint32_t heads,
+                       uint32_t kheads, uint32_t head_dim, uint32_t base, uint32_t rows, const void* pos_ptr) {
     if (!t.table) return fail(b, GH_E_STATE, "rope: table not built");
     GhRopeArgs a{};
-    a.x = x->addr;
+    a.x = q ? q->addr : 0;
+    a.k = k ? k->addr : 0;
     a.table = (uint64_t)t.table;
-    a.post = role == GH_ROPE_QUERY ? (uint64_t)t.post : 0;
+    a.post = (uint64_t)t.post;
     a.pos_ptr = (uint64_t)pos_ptr;
-    a.heads = heads;
+    a.heads = q ? heads : 0;
+    a.kheads = k ? kheads : 0;
     a.head_dim = head_dim;
     a.pairs = t.yarn.rope_dim / 2;
     a.base = base;
     a.rows = rows;
-    uint64_t total = (uint64_t)rows * heads * a.pairs;
-    return launch(b, K_ROPE, ceil_div(total, 256), 1, 1, 256, &a);
+    // four pairs per thread: 16-byte loads of the values and of the table
+    a.per = a.pairs % 4 == 0 && head_dim % 8 == 0 && a.x % 16 == 0 && a.k % 16 == 0 ? 4 : 1;
+    a.groups = ceil_div((uint64_t)(a.heads + a.kheads) * (a.pairs / a.per), 256);
+    if (rows == 0 || a.groups == 0) return GH_OK;
+    if ((uint64_t)rows * a.groups > 0x7FFFFFFFull) return fail(b, GH_E_RANGE, "rope: too many rows");
+    return launch(b, K_ROPE, rows * a.groups, 1, 1, 256, &a);
+}
+
+int op_rope(gh_backend* b, const GhRopeTable& t, const gh_buf* x, uint32_t heads,
+            uint32_t head_dim, uint32_t base, uint32_t rows, uint32_t role, const void* pos_ptr) {
+    const bool query = role == GH_ROPE_QUERY;
+    return rope_launch(b, t, query ? x : nullptr, query ? nullptr : x, heads, heads, head_dim, base, rows, pos_ptr);
 }
 
 int op_kv_write(gh_backend* b, const gh_kv* kv, const gh_buf* k, const gh_buf* v,
@@ -287,7 +300,9 @@ int op_kv_write(gh_backend* b, const gh_kv* kv, const gh_buf* k, const gh_buf* v
     a.v_count = vectors * kv->value_dim;
     a.k_stride = kv->kv_heads * kv->head_dim;
     a.v_stride = kv->kv_heads * kv->value_dim;
-    return launch(b, K_KV_WRITE, ceil_div(std::max(a.k_count, a.v_count), 256), 1, 1, 256, &a);
+    a.wide = (a.kc | a.vc | a.k | a.v) % 16 == 0 && (a.k_off | a.v_off) % 8 == 0 &&
+             (!pos_ptr || (a.k_stride | a.v_stride) % 8 == 0);
+    return launch(b, K_KV_WRITE, ceil_div(std::max(a.k_count, a.v_count), 2048), 1, 1, 256, &a);
 }
 
 // Workgroups per (row, kv head): enough that rows x kv heads x splits covers about two
@@ -1140,6 +1155,7 @@ static int gemm_kernel(gh_backend* b, const GemmPlan& p, uint64_t out, uint64_t 
 // epilogue (in the GEMM or the reduce) or replaces the reduce by gh_gemm_tail (residual add
 // and RMSNorm of each output row).
 int op_gemm(gh_backend* b, uint64_t out, const gh_buf* a, const gh_buf* w, uint32_t n, const GemmEpi* e) {
+    if (n < 8 && w->cols > 16384) return fail(b, GH_E_UNSUPPORTED, "gemv: in_dim above 16384");
     const GemmPlan p = plan_gemm(b, w, n);
     const bool tail = e && e->resid;
     const uint32_t epi = e && !tail ? e->epi : GH_GEMM_EPI_F16;
@@ -1389,6 +1405,10 @@ int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint3
         return launch(b, K_GEMM_REDUCE_SEG, (uint32_t)std::min<uint64_t>(ceil_div(npairs, (uint64_t)256), 4096), 1, 1,
                       256, &ga);
     }
+    if (nseg >= 2 && segs[0].role == GH_GEMM_ROLE_ROPE_QUERY && segs[1].role == GH_GEMM_ROLE_ROPE_KEY &&
+        (nseg < 3 || !segs[2].role))
+        return rope_launch(b, *rope, segs[0].out, segs[1].out, segs[0].w->rows / head_dim, segs[1].w->rows / head_dim,
+                           head_dim, base, n, nullptr);
     for (uint32_t i = 0; i < nseg && !rc; ++i)
         if (segs[i].role)
             rc = op_rope(b, *rope, segs[i].out, segs[i].w->rows / head_dim, head_dim, base, n,
@@ -1423,7 +1443,6 @@ static int gemv_launch(gh_backend* b, const gh_buf* out, const gh_buf* a, const 
     if (w->cols != in_dim || w->rows != out_dim) return fail(b, GH_E_INVALID, "matmul: weight shape mismatch");
     if (!fits(a, (uint64_t)n * in_dim * 2) || !fits(out, (uint64_t)n * out_dim * (f32 ? 4 : 2)))
         return fail(b, GH_E_RANGE, "matmul: buffer too small");
-    if (in_dim / 64 > 256 && n < 8) return fail(b, GH_E_UNSUPPORTED, "gemv: in_dim above 16384");
     // Fewer than 8 tokens of a small matrix: the GEMV reads it once per token, mostly from the caches,
     // without the GEMM's split reduce (about 2.5 us + 0.3 us per MB and token against 9.5 + 0.14 per MB:
     // 4096 x 4096 Q4_K at 2 / 5 tokens 8.3 / 16.1 us against 9.6 / 10.2, 1024 x 4096 Q6_K 4.9 / 8.6
@@ -1491,8 +1510,7 @@ int gh_rope_yarn_batched(gh_backend* b, gh_encoder* enc, const gh_buf* q, const 
     if (!fits(q, (uint64_t)rows * q_heads * head_dim * 2) || !fits(k, (uint64_t)rows * kv_heads * head_dim * 2))
         return latch(enc, fail(b, GH_E_RANGE, "rope: buffer too small"));
     rc = ensure_rope(b, b->rope, yarn, base + rows);
-    if (!rc) rc = op_rope(b, b->rope, q, q_heads, head_dim, base, rows, GH_ROPE_QUERY, nullptr);
-    if (!rc) rc = op_rope(b, b->rope, k, kv_heads, head_dim, base, rows, GH_ROPE_KEY, nullptr);
+    if (!rc) rc = rope_launch(b, b->rope, q, k, q_heads, kv_heads, head_dim, base, rows, nullptr);
     return latch(enc, rc);
 }
 
@@ -1502,8 +1520,8 @@ int gh_silu_mul(gh_backend* b, gh_encoder* enc, const gh_buf* out, const gh_buf*
     if (rc) return rc;
     if (!fits(out, (uint64_t)n * 2) || !fits(gate, (uint64_t)n * 2) || !fits(up, (uint64_t)n * 2))
         return latch(enc, fail(b, GH_E_RANGE, "silu_mul: buffer too small"));
-    GhEltArgs a{out->addr, gate->addr, up->addr, n, 0};
-    return latch(enc, launch(b, K_SILU_MUL, ceil_div(n, 256), 1, 1, 256, &a));
+    GhEltArgs a{out->addr, gate->addr, up->addr, n, (out->addr | gate->addr | up->addr) % 16 == 0};
+    return latch(enc, launch(b, K_SILU_MUL, ceil_div(n, 2048), 1, 1, 256, &a));
 }
 
 int gh_residual_add(gh_backend* b, gh_encoder* enc, const gh_buf* x, const gh_buf* y,
@@ -1512,8 +1530,8 @@ int gh_residual_add(gh_backend* b, gh_encoder* enc, const gh_buf* x, const gh_bu
     if (rc) return rc;
     if (!fits(x, (uint64_t)n * 4) || !fits(y, (uint64_t)n * 2))
         return latch(enc, fail(b, GH_E_RANGE, "residual_add: buffer too small"));
-    GhEltArgs a{x->addr, 0, y->addr, n, 0};
-    return latch(enc, launch(b, K_RESIDUAL_ADD, ceil_div(n, 256), 1, 1, 256, &a));
+    GhEltArgs a{x->addr, 0, y->addr, n, (x->addr | y->addr) % 16 == 0};
+    return latch(enc, launch(b, K_RESIDUAL_ADD, ceil_div(n, 2048), 1, 1, 256, &a));
 }
 
 

@@ -149,20 +149,23 @@ struct GhRmsnormArgs {
     uint32_t pad;
 };
 
-// RoPE over `rows` packed rows of `heads` heads; row r sits at absolute position base + r (or
-// base + *pos_ptr when pos_ptr != 0). table: float2 (cos, sin) [positions][pairs];
-// post: f32 [positions] query post-scale (role 0) — 1.0 for keys.
+// RoPE over `rows` packed rows of `heads` query heads (post: f32 [positions] query post-scale; 0: 1.0)
+// and of `kheads` key heads; row r sits at absolute position base + r (or base + *pos_ptr when
+// pos_ptr != 0). table: float2 (cos, sin) [positions][pairs].
 struct GhRopeArgs {
     uint64_t x;       // f16 [rows][heads][head_dim], rotated in place
+    uint64_t k;       // f16 [rows][kheads][head_dim], rotated in place without post-scale
     uint64_t table;
-    uint64_t post;    // 0 for keys
+    uint64_t post;
     uint64_t pos_ptr; // optional u32* position on the device
     uint32_t heads;
+    uint32_t kheads;
     uint32_t head_dim;
     uint32_t pairs;   // rope_dim / 2
     uint32_t base;
     uint32_t rows;
-    uint32_t pad;
+    uint32_t per;     // pairs per thread: 4 (16-byte accesses) or 1
+    uint32_t groups;  // workgroups per row
 };
 
 struct GhEltArgs {
@@ -170,7 +173,7 @@ struct GhEltArgs {
     uint64_t a;
     uint64_t b;
     uint32_t n;
-    uint32_t pad;
+    uint32_t pad;   // silu_mul, residual_add: 16-byte accesses allowed; else the kernel's own
 };
 
 // KV append of `vectors_k` K values (and V) at element offsets (off + pos*stride) when pos_ptr.
@@ -186,6 +189,8 @@ struct GhKvWriteArgs {
     uint32_t v_count;
     uint32_t k_stride;   // elements per position (pos_ptr mode)
     uint32_t v_stride;
+    uint32_t wide;       // 16-byte accesses allowed
+    uint32_t pad;
 };
 
 // Split-K flash decode: grid (splits, kv_heads, rows). Row r attends positions 0..pos_r where

@@ -1,9 +1,11 @@
 // Decode/prefill glue: RMSNorm, YaRN RoPE, SiLU·up, residual add, KV append, argmax.
 #include "gh_common.h"
 
-// rmsnorm_x (backend/cpu/kernels/elementwise/normalization.rs:12-40): one 1024-thread
-// workgroup per row, 4 consecutive FP32 values per thread per step, Σx² reduced with DPP and
-// LDS, inverse = 1/sqrt(Σx²/dim + eps), out = f16((x*inverse)*w). dim % 4 == 0.
+// rmsnorm_x (backend/cpu/kernels/elementwise/normalization.rs:12-40): one 256-thread
+// workgroup per row, Σx² in gh_rms_inverse_256's order (thread t: the 16-value items t, t + 256, ...),
+// inverse = 1/sqrt(Σx²/dim + eps), out = f16((x*inverse)*w). dim % 4 == 0. Bound by memory (x in, out
+// out): rows of up to 8192 values stay in registers between the sum and the scaling (2000 x 4096 read
+// twice 15.2 us, now 12.6).
 GH_KERNEL __launch_bounds__(256) void gh_rmsnorm_x(GhRmsnormArgs a) {
 #pragma clang fp contract(off)
     const uint32_t row = blockIdx.x;
@@ -12,54 +14,118 @@ GH_KERNEL __launch_bounds__(256) void gh_rmsnorm_x(GhRmsnormArgs a) {
     const GH_GLOBAL uint2* w = gh_gp<uint2>(a.w);
     GH_GLOBAL uint2* out = gh_gpw<uint2>(a.out + (uint64_t)row * a.dim * 2);
     __shared__ float red[4];
-    const float inverse = gh_rms_inverse_256(x, a.dim, a.eps, red);
-    for (uint32_t i = threadIdx.x; i < (a.dim >> 2); i += 256) {
-        const float4 v = x[i];
+    const uint32_t n4 = a.dim >> 2;
+    auto scaled = [&](const float4& v, float inverse, uint32_t i) __attribute__((always_inline)) {
         const uint2 wv = w[i];
         const uint32_t o0 = gh_f2h(v.x * inverse * gh_h2f(wv.x & 0xFFFFu));
         const uint32_t o1 = gh_f2h(v.y * inverse * gh_h2f(wv.x >> 16));
         const uint32_t o2 = gh_f2h(v.z * inverse * gh_h2f(wv.y & 0xFFFFu));
         const uint32_t o3 = gh_f2h(v.w * inverse * gh_h2f(wv.y >> 16));
         out[i] = make_uint2(o0 | (o1 << 16), o2 | (o3 << 16));
+    };
+    if (a.dim > 8192) {
+        const float inverse = gh_rms_inverse_256(x, a.dim, a.eps, red);
+        for (uint32_t i = threadIdx.x; i < n4; i += 256) scaled(x[i], inverse, i);
+        return;
     }
+    float4 v[2][4];
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k)
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) v[k][q] = x[min(4 * (threadIdx.x + 256 * k) + q, n4 - 1)];
+    float s = 0.0f;
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k)
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q)
+            if (4 * (threadIdx.x + 256 * k) + q < n4) s = gh_rms_add(s, v[k][q]);
+    const float inverse = gh_rms_finish_256(s, a.dim, a.eps, red);
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k)
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint32_t i = 4 * (threadIdx.x + 256 * k) + q;
+            if (i < n4) scaled(v[k][q], inverse, i);
+        }
+}
+
+// One pair of RoPE: (x0, x1) in v rotated by cs, times the post-scale
+__device__ __forceinline__ uint32_t rope_pair(uint32_t v, float c, float s, float scale) {
+#pragma clang fp contract(off)
+    const float x0 = gh_h2f(v & 0xFFFFu), x1 = gh_h2f(v >> 16);
+    const float y0 = (x0 * c - x1 * s) * scale;
+    const float y1 = (x0 * s + x1 * c) * scale;
+    return (uint32_t)gh_f2h(y0) | ((uint32_t)gh_f2h(y1) << 16);
 }
 
 // rope_yarn (cpu/kernels/elementwise/rope.rs:14-39): adjacent pairs rotated by the per
-// (position, pair) YaRN (cos, sin) table, then the role's post-scale; FP16 in place.
-// One thread per (row, head, pair).
+// (position, pair) YaRN (cos, sin) table, then the role's post-scale; FP16 in place. Query heads
+// and, in the same launch, key heads (no post-scale). a.groups workgroups per row, a thread per a.per
+// pairs: four (16 bytes) where the head and the addresses allow it, else one (a row of 32 + 8 heads
+// in two launches of one pair per thread took 13.5 + 4.7 us at 2000 rows, now
+// 9.9).
 GH_KERNEL __launch_bounds__(256) void gh_rope(GhRopeArgs a) {
-#pragma clang fp contract(off)
-    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t total = (size_t)a.rows * a.heads * a.pairs;
-    if (t >= total) return;
-    const uint32_t pair = (uint32_t)(t % a.pairs);
-    const size_t rh = t / a.pairs;
-    const uint32_t head = (uint32_t)(rh % a.heads);
-    const uint32_t row = (uint32_t)(rh / a.heads);
-    const uint32_t pos = (a.pos_ptr ? *(const uint32_t*)a.pos_ptr : 0u) + a.base + row;
-    const float2 cs = ((const float2*)a.table)[(size_t)pos * a.pairs + pair];
-    const float scale = a.post ? ((const float*)a.post)[pos] : 1.0f;
-    uint32_t* p = (uint32_t*)((uint16_t*)a.x + ((size_t)row * a.heads + head) * a.head_dim + 2 * pair);
-    const uint32_t v = *p;
-    const float x0 = gh_h2f(v & 0xFFFFu), x1 = gh_h2f(v >> 16);
-    const float y0 = (x0 * cs.x - x1 * cs.y) * scale;
-    const float y1 = (x0 * cs.y + x1 * cs.x) * scale;
-    *p = (uint32_t)gh_f2h(y0) | ((uint32_t)gh_f2h(y1) << 16);
+    const uint32_t row = blockIdx.x / a.groups;  // workgroup-uniform
+    const uint32_t t = (blockIdx.x % a.groups) * 256 + threadIdx.x, quads = a.pairs / a.per;
+    uint32_t head = t / quads;
+    const uint32_t pair = (t % quads) * a.per;
+    if (head >= a.heads + a.kheads) return;
+    const uint32_t pos = (a.pos_ptr ? *gh_gp<uint32_t>(a.pos_ptr) : 0u) + a.base + row;
+    const bool key = head >= a.heads;
+    if (key) head -= a.heads;
+    const float scale = !key && a.post ? gh_gp<float>(a.post)[pos] : 1.0f;
+    const uint64_t p = (key ? a.k : a.x) + (((uint64_t)row * (key ? a.kheads : a.heads) + head) * a.head_dim + 2 * pair) * 2;
+    const uint64_t cs = a.table + ((uint64_t)pos * a.pairs + pair) * 8;
+    if (a.per == 4) {
+        const uint4 v = *gh_gp<uint4>(p);
+        const float4 c0 = *gh_gp<float4>(cs), c1 = *gh_gp<float4>(cs + 16);
+        *gh_gpw<uint4>(p) = make_uint4(rope_pair(v.x, c0.x, c0.y, scale), rope_pair(v.y, c0.z, c0.w, scale),
+                                       rope_pair(v.z, c1.x, c1.y, scale), rope_pair(v.w, c1.z, c1.w, scale));
+    } else {
+        const float2 c = *gh_gp<float2>(cs);
+        *gh_gpw<uint32_t>(p) = rope_pair(*gh_gp<uint32_t>(p), c.x, c.y, scale);
+    }
 }
 
+// The elementwise kernels below take 8 consecutive values per thread: 16-byte accesses where a.pad
+// says that every address allows them (2-byte ones ran silu_mul of 24.6 M values at 3.0 TB/s, 50 us; now
+// 26.2 us, 5.6 TB/s; kv_write of 2000 x 2 x 1024 values 7.0 -> 4.2), value by value otherwise and in the
+// last, partial thread.
 // silu_mul (cpu/kernels/elementwise/activation.rs:16-29): out = f16(f16(g/(1+exp(-g))) * u).
 GH_KERNEL __launch_bounds__(256) void gh_silu_mul(GhEltArgs a) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= a.n) return;
-    ((uint16_t*)a.out)[i] = gh_silu_mul_h(((const uint16_t*)a.a)[i], ((const uint16_t*)a.b)[i]);
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (a.pad && i + 8 <= a.n) {
+        const uint4 g = *gh_gp<uint4>(a.a + 2 * i), u = *gh_gp<uint4>(a.b + 2 * i);
+        auto two = [](uint32_t g2, uint32_t u2) __attribute__((always_inline)) {
+            return (uint32_t)gh_silu_mul_h(g2 & 0xFFFFu, u2 & 0xFFFFu) | ((uint32_t)gh_silu_mul_h(g2 >> 16, u2 >> 16) << 16);
+        };
+        *gh_gpw<uint4>(a.out + 2 * i) = make_uint4(two(g.x, u.x), two(g.y, u.y), two(g.z, u.z), two(g.w, u.w));
+        return;
+    }
+    for (size_t k = i; k < a.n && k < i + 8; ++k)
+        gh_gpw<uint16_t>(a.out)[k] = gh_silu_mul_h(gh_gp<uint16_t>(a.a)[k], gh_gp<uint16_t>(a.b)[k]);
 }
 
 // residual_add (cpu/kernels/elementwise/residual.rs:12-22): x(f32) += f16 y.
 GH_KERNEL __launch_bounds__(256) void gh_residual_add(GhEltArgs a) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= a.n) return;
-    float* x = (float*)a.out;
-    x[i] = x[i] + gh_h2f(((const uint16_t*)a.b)[i]);
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (a.pad && i + 8 <= a.n) {
+        GH_GLOBAL float4* x = gh_gpw<float4>(a.out + 4 * i);
+        const uint4 y = *gh_gp<uint4>(a.b + 2 * i);
+        float4 u = x[0], v = x[1];
+        u.x += gh_h2f(y.x & 0xFFFFu);
+        u.y += gh_h2f(y.x >> 16);
+        u.z += gh_h2f(y.y & 0xFFFFu);
+        u.w += gh_h2f(y.y >> 16);
+        v.x += gh_h2f(y.z & 0xFFFFu);
+        v.y += gh_h2f(y.z >> 16);
+        v.z += gh_h2f(y.w & 0xFFFFu);
+        v.w += gh_h2f(y.w >> 16);
+        x[0] = u;
+        x[1] = v;
+        return;
+    }
+    for (size_t k = i; k < a.n && k < i + 8; ++k) gh_gpw<float>(a.out)[k] += gh_h2f(gh_gp<uint16_t>(a.b)[k]);
 }
 
 // Fill n u32 words at `out` with the value `pad`: a clear that a captured graph records as a
@@ -97,12 +163,17 @@ GH_KERNEL __launch_bounds__(256) void gh_stream_probe(GhEltArgs a) {
 // kv_write f16 (cpu/kernels/attention/write.rs:50-63): raw FP16 copy of K and V into the
 // caches at element offsets; with pos_ptr the offsets advance by stride * (*pos_ptr).
 GH_KERNEL __launch_bounds__(256) void gh_kv_write(GhKvWriteArgs a) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t pos = a.pos_ptr ? *(const uint32_t*)a.pos_ptr : 0u;
-    if (i < a.k_count)
-        ((uint16_t*)a.kc)[a.k_off + pos * a.k_stride + i] = ((const uint16_t*)a.k)[i];
-    if (i < a.v_count)
-        ((uint16_t*)a.vc)[a.v_off + pos * a.v_stride + i] = ((const uint16_t*)a.v)[i];
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    const size_t pos = a.pos_ptr ? *gh_gp<uint32_t>(a.pos_ptr) : 0u;
+    auto copy = [&](uint64_t dst, uint64_t src, uint32_t count) __attribute__((always_inline)) {
+        if (a.wide && i + 8 <= count) {
+            *gh_gpw<uint4>(dst + 2 * i) = *gh_gp<uint4>(src + 2 * i);
+            return;
+        }
+        for (size_t k = i; k < count && k < i + 8; ++k) gh_gpw<uint16_t>(dst)[k] = gh_gp<uint16_t>(src)[k];
+    };
+    copy(a.kc + 2 * (a.k_off + pos * a.k_stride), a.k, a.k_count);
+    copy(a.vc + 2 * (a.v_off + pos * a.v_stride), a.v, a.v_count);
 }
 
 // argmax_f32 (backend/cpu/readback.rs:45-55): first index of the maximum, NaN never wins;

@@ -7,6 +7,7 @@ Bars (stated per test):
   * FP16 glue with a transcendental or a reduction (silu_mul, rmsnorm): within 1 FP16 ulp.
 """
 import math
+from dataclasses import replace
 
 import numpy as np
 import pytest
@@ -223,6 +224,76 @@ def test_silu_mul_within_one_ulp(hip):
     assert d.max() <= 1 and (d == 0).mean() > 0.99
     for b in (gb, ub, ob):
         hip.free_buffer(b)
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 2049, 4104])
+@pytest.mark.parametrize("shift", [0, 2], ids=["aligned", "unaligned"])
+def test_elementwise_ops_wide_and_narrow(hip, n, shift):
+    """silu_mul, residual_add and kv_write with 16-byte accesses and, where an address or an offset
+    does not allow them, value by value: the same bytes, and nothing past the end."""
+    rng = np.random.default_rng(n)
+    g, u = (O.f16(rng.standard_normal(n + 8).astype(np.float32)) for _ in range(2))
+    x = rng.standard_normal(n + 8).astype(np.float32)
+
+    def at(buf, size):  # a handle `shift` values into the buffer
+        return F.GhBuf(buf.addr + shift * size, buf.bytes - shift * size, buf.format, F.BUF_VIEW, 0, 0)
+
+    gb, ub, xb, ob = hip.from_host(g), hip.from_host(u), hip.from_host(x), hip.from_host(np.full(n + 8, 0x1234, np.uint16))
+    hip.silu_mul(at(ob, 2), at(gb, 2), at(ub, 2), n)
+    out = hip.download(ob, np.uint16, n + 8)
+    ref = hip.from_host(np.zeros(n, np.uint16))
+    for i in range(0, n, max(1, n // 16)):  # one value at a time: always the narrow form
+        hip.silu_mul(F.GhBuf(ref.addr + 2 * i, 2, F.FMT_F16, F.BUF_VIEW, 0, 0),
+                     F.GhBuf(gb.addr + 2 * (shift + i), 2, F.FMT_F16, F.BUF_VIEW, 0, 0),
+                     F.GhBuf(ub.addr + 2 * (shift + i), 2, F.FMT_F16, F.BUF_VIEW, 0, 0), 1)
+        assert hip.download(ref, np.uint16, 1, offset=2 * i)[0] == out[shift + i]
+    assert (out[:shift] == 0x1234).all() and (out[shift + n:] == 0x1234).all()
+    hip.residual_add(at(xb, 4), at(gb, 2), n)
+    got = hip.download(xb, np.float32, n + 8)
+    want = x.copy()
+    want[shift:shift + n] += O.f32(g)[shift:shift + n]
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    for b in (gb, ub, xb, ob, ref):
+        hip.free_buffer(b)
+    vectors, off = 5, shift  # kv_write at a cache offset that is (not) a multiple of 16 bytes
+    k, v = (O.f16(rng.standard_normal(vectors * 128).astype(np.float32)) for _ in range(2))
+    kb, vb = hip.from_host(k), hip.from_host(v)
+    kc, vc = (hip.from_host(np.zeros(8 * 256, np.uint16)) for _ in range(2))
+    kv = F.GhKv(kc, vc, F.KV_F16, 1, 8, 2, 128, 128)
+    hip.kv_write(kv, kb, vb, 2 * (256 + off), 2 * (384 + off), vectors)
+    for cache, src, o in ((kc, k, 256 + off), (vc, v, 384 + off)):
+        want = np.zeros(8 * 256, np.uint16)
+        want[o:o + vectors * 128] = src
+        assert np.array_equal(hip.download(cache, np.uint16, 8 * 256), want)
+    for b in (kb, vb, kc, vc):
+        hip.free_buffer(b)
+
+
+@pytest.mark.parametrize("rope_dim,heads,kheads,rows,shift", [(128, 4, 2, 3, 0), (24, 3, 1, 5, 0), (64, 5, 3, 70, 0),
+                                                              (10, 2, 2, 4, 0), (128, 32, 8, 2, 2), (128, 70, 9, 3, 0)])
+def test_rope_batched_widths(hip, rope_dim, heads, kheads, rows, shift):
+    """Rotations four pairs at a time and one at a time (a pair count that is no multiple of four, an
+    address that is no multiple of 16), queries and keys in one launch: the bits of the oracle's rows.
+    (Positions below 16384: above, the kernel rounds the product with the post-scale once, to FP16,
+    where the oracle rounds it to FP32 first, which differs on about one value in 10^5.)"""
+    rng = np.random.default_rng(rope_dim + rows)
+    q, k = (O.f16(rng.standard_normal(rows * h * 128 + 8).astype(np.float32)) for h in (heads, kheads))
+    qb, kb = hip.from_host(q), hip.from_host(k)
+
+    def at(buf):
+        return F.GhBuf(buf.addr + 2 * shift, buf.bytes - 2 * shift, buf.format, F.BUF_VIEW, 0, 0)
+
+    base = 16000
+    oy = O.Yarn(rope_dim, 16384, 1e6, 16.0, 32.0, 1.0, 1.0, 0.1)
+    hip.rope_yarn_batched(at(qb), at(kb), heads, kheads, 128, base, rows, replace(YARN, rope_dim=rope_dim))
+    for buf, src, h, role in ((qb, q, heads, F.ROPE_QUERY), (kb, k, kheads, F.ROPE_KEY)):
+        got = hip.download(buf, np.uint16, len(src))
+        want = src.copy()
+        for r in range(rows):
+            a = shift + r * h * 128
+            want[a:a + h * 128] = O.rope_yarn(src[a:a + h * 128], h, 128, base + r, oy, role)
+        assert np.array_equal(got, want), (rope_dim, role)
+        hip.free_buffer(buf)
 
 
 def test_residual_add_bit_exact(hip):
