@@ -90,6 +90,7 @@ const char* kModules[] = {"gh_quant", "gh_gemv", "gh_glue", "gh_attention", "gh_
 constexpr uint32_t kArgmaxBlocks = 256;
 // argmax scratch at the front of the workspace: f32[256] values, u32[256] indices, u32 result
 constexpr size_t kArgmaxBytes = 256 * 4 * 2 + 256;
+constexpr size_t kResultBytes = 2 * 128 * 4;  // read_argmax's index, or read_topk's 128 indices and values
 
 std::string library_dir() {
     Dl_info info{};
@@ -812,6 +813,7 @@ int gh_create(const gh_config* cfg, gh_backend** out) {
     // hipGetLastError after its own calls) would take for its own failure
     (void)hipGetLastError();
     if (!rc) rc = ensure_workspace(b, 0);
+    if (!rc) rc = hip_check(b, hipHostMalloc((void**)&b->result, kResultBytes, hipHostMallocDefault), "hipHostMalloc");
     if (!rc) rc = noalloc_init(b);
     if (!rc) {
         b->xcds = probe_xcds(b);
@@ -830,6 +832,7 @@ void gh_destroy(gh_backend* b) {
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     if (b->ws) (void)hipFree(b->ws);
     if (b->counters) (void)hipFree(b->counters);
+    if (b->result) (void)hipHostFree(b->result);
     free_rope(b->rope);
     for (hipModule_t m : b->modules) (void)hipModuleUnload(m);
     if (b->ev_start) (void)hipEventDestroy(b->ev_start);
@@ -1565,18 +1568,17 @@ int gh_read_argmax(gh_backend* b, const gh_buf* logits, uint64_t vocab, uint32_t
     if (!b || !logits || !out) return GH_E_INVALID;
     if (vocab == 0) return fail(b, GH_E_INVALID, "read_argmax on empty logits");
     if (!fits(logits, vocab * 4)) return fail(b, GH_E_RANGE, "read_argmax: buffer smaller than vocab");
-    int rc = op_argmax(b, logits, vocab, nullptr, nullptr);
-    if (rc) return rc;
-    rc = hip_check(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-    if (rc) return rc;
-    return hip_check(b, hipMemcpy(out, (char*)b->ws + 2048, 4, hipMemcpyDeviceToHost), "hipMemcpy argmax");
+    int rc = op_argmax(b, logits, vocab, b->result, nullptr);  // into pinned host memory
+    if (!rc) rc = hip_check(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+    if (!rc) *out = *b->result;
+    return rc;
 }
 
 // read_topk: k <= 128 on the device (gh_topk_partial over stripes of at most kTopkChunk
 // logits per step, at most 128 stripes, then gh_topk_final; 8 k bytes come back), larger k
 // on the host over the read-back logits. Both give exactly the reference's selection and
 // order (cpu/readback.rs:59-69): (logit desc by f32 total order, index asc).
-constexpr uint64_t kTopkDeviceMax = 128, kTopkChunk = 2048, kTopkStripes = 128;
+constexpr uint64_t kTopkDeviceMax = 128, kTopkChunk = 512, kTopkStripes = 256;
 
 int gh_read_topk(gh_backend* b, const gh_buf* logits, uint64_t vocab, uint64_t k, uint32_t* idx,
                  float* val, uint64_t* count) {
@@ -1588,9 +1590,8 @@ int gh_read_topk(gh_backend* b, const gh_buf* logits, uint64_t vocab, uint64_t k
     *count = 0;
     if (k == 0) return GH_OK;
     if (k <= kTopkDeviceMax) {
-        uint32_t width = 1;
-        while (width < k) width <<= 1;
-        // stripes of kTopkChunk logits, widened (in whole chunks) to keep at most 128 stripes
+        const uint32_t width = k <= 64 ? 64 : 128;
+        // stripes of kTopkChunk logits, widened (in whole chunks) to keep at most kTopkStripes
         const uint64_t chunks = (vocab + kTopkChunk - 1) / kTopkChunk;
         const uint64_t per = kTopkChunk * ((chunks + kTopkStripes - 1) / kTopkStripes);
         GhTopkArgs a{};
@@ -1600,19 +1601,15 @@ int gh_read_topk(gh_backend* b, const gh_buf* logits, uint64_t vocab, uint64_t k
         a.stripes = (uint32_t)((vocab + per - 1) / per);
         a.width = width;
         a.k = (uint32_t)k;
-        const size_t part_bytes = (size_t)a.stripes * width * 8;
-        int rc = ensure_workspace(b, part_bytes + 8 * k);
+        int rc = ensure_workspace(b, (size_t)a.stripes * width * 8);
         if (rc) return rc;
-        char* ws = (char*)b->ws + kArgmaxBytes;
-        a.part = (uint64_t)ws;
-        a.out = (uint64_t)(ws + part_bytes);
-        rc = launch(b, K_TOPK_PARTIAL, a.stripes, 1, 1, 512, &a);
+        a.part = (uint64_t)((char*)b->ws + kArgmaxBytes);
+        a.out = (uint64_t)b->result;  // pinned host memory: no copy after the kernel
+        rc = launch(b, K_TOPK_PARTIAL, a.stripes, 1, 1, 64, &a);
         if (!rc) rc = launch(b, K_TOPK_FINAL, 1, 1, 1, 1024, &a);
         if (!rc) rc = hip_check(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-        std::vector<uint32_t> pairs(2 * k);
-        if (!rc) rc = hip_check(b, hipMemcpy(pairs.data(), ws + part_bytes, 8 * k, hipMemcpyDeviceToHost),
-                                "hipMemcpy topk");
         if (rc) return rc;
+        const uint32_t* pairs = b->result;
         for (uint64_t i = 0; i < k; ++i) {
             if (idx) idx[i] = pairs[i];
             if (val) std::memcpy(&val[i], &pairs[k + i], 4);

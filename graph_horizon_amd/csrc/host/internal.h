@@ -159,6 +159,7 @@ struct gh_backend {
     std::string err;
     // growable device workspace (attention partials, argmax partials)
     void* ws = nullptr;
+    uint32_t* result = nullptr;  // pinned host memory that the read-back kernels write
     size_t ws_bytes = 0;
     void* counters = nullptr;  // attention merge counters, zero between launches
     size_t counter_slots = 0;

@@ -222,7 +222,7 @@ struct GhAttnArgs {
 
 // Device top-k (read_topk): gh_topk_partial keeps the `width` smallest keys of each stripe of
 // `per` logits (grid = stripes); gh_topk_final merges the stripes' lists and writes the first
-// k as (u32 index, f32 bits) pairs.
+// k as u32 indices, then f32 bits.
 struct GhTopkArgs {
     uint64_t logits;   // f32 [n]
     uint64_t part;     // u64 keys [stripes][width]
@@ -230,7 +230,7 @@ struct GhTopkArgs {
     uint32_t n;
     uint32_t per;      // logits per stripe
     uint32_t stripes;
-    uint32_t width;    // power of 2 >= k, <= 128
+    uint32_t width;    // 64 (k <= 64) or 128
     uint32_t k;
 };
 

@@ -249,97 +249,184 @@ GH_KERNEL __launch_bounds__(256) void gh_argmax_final(GhArgmaxArgs a) {
 // ascending in exactly that order:
 //   key = (~ord(bits) << 32) | index,   ord(b) = b ^ (b >> 31 ? 0xFFFFFFFF : 0x80000000),
 // ord mapping the total order of f32 bit patterns (-NaN < -inf < ... < -0 < +0 < ... < +inf <
-// +NaN) onto unsigned order. The all-ones key pads short stripes and sorts after every real
-// key. Both kernels sort with bitonic networks in LDS.
-constexpr uint32_t kTopkChunk = 2048;  // keys sorted per step of the partial pass
-constexpr uint32_t kTopkWidth = 128;   // largest list width (k <= 128 on the device path)
-constexpr uint32_t kTopkStripes = 128; // largest stripe count
+// +NaN) onto unsigned order. The all-ones key pads short stripes and lists and sorts after every
+// real key.
+// Everything is a sorted list of 64·V keys (V = 1 up to k = 64, else 2) in the registers of one
+// wave, entry 64 v + lane in register v: bitonic networks over lane exchanges, no LDS and no barrier
+// between their steps (sorted 2048 at a time in LDS by eight waves, 66 barriers, a stripe took 23 us
+// and the merge of the 64 stripes 12.5; now 8.4 and 11.3 at 131072 logits and k = 40 with the result
+// written to pinned host memory, one call in all 58.4 -> 31.5 us). Two lists of opposite directions merge by
+// min(A[i], B[i]), which holds the smallest half as a bitonic list.
+constexpr uint32_t kTopkChunk = 512;   // keys a wave sorts at a time (8 registers)
 
 __device__ __forceinline__ uint64_t topk_key(uint32_t bits, uint32_t idx) {
     const uint32_t ord = bits ^ ((bits >> 31) ? 0xFFFFFFFFu : 0x80000000u);
     return ((uint64_t)~ord << 32) | idx;
 }
 
-// Ascending bitonic sort of s[0, n), n a power of 2, by the whole workgroup.
-template <uint32_t NT>
-__device__ void topk_sort(uint64_t* s, uint32_t n) {
-    for (uint32_t size = 2; size <= n; size <<= 1) {
-        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-            __syncthreads();
-            for (uint32_t t = threadIdx.x; t < n / 2; t += NT) {
-                const uint32_t i = 2 * t - (t & (stride - 1)), j = i + stride;
-                const uint64_t x = s[i], y = s[j];
-                if ((x > y) == ((i & size) == 0)) {
-                    s[i] = y;
-                    s[j] = x;
-                }
-            }
-        }
+// The smaller (keep_min) or larger of x and lane ^ stride's x: DPP moves within 16 lanes (xor 4 as
+// xor 7 then xor 3), row swaps beyond, which leave the lane's own and its partner's value in the two
+// registers (through ds_bpermute: partial 13.5 us, final 13.9 at k = 40).
+template <int CTRL>
+__device__ __forceinline__ uint64_t topk_dpp(uint64_t x) {
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, 0xF, 0xF, false);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, 0xF, 0xF, false);
+    return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ uint64_t topk_exchange(uint64_t x, uint32_t stride, bool keep_min) {
+    uint64_t y;
+    if (stride >= 16) {
+        const uint32_t l = (uint32_t)x, h = (uint32_t)(x >> 32);
+        const auto a = stride == 16 ? __builtin_amdgcn_permlane16_swap(l, l, false, false)
+                                    : __builtin_amdgcn_permlane32_swap(l, l, false, false);
+        const auto b = stride == 16 ? __builtin_amdgcn_permlane16_swap(h, h, false, false)
+                                    : __builtin_amdgcn_permlane32_swap(h, h, false, false);
+        x = ((uint64_t)b[0] << 32) | a[0];
+        y = ((uint64_t)b[1] << 32) | a[1];
+    } else if (stride == 8) {
+        y = topk_dpp<0x128>(x);  // row_ror:8
+    } else if (stride == 4) {
+        y = topk_dpp<0x1B>(topk_dpp<0x141>(x));  // row_half_mirror, quad_perm [3,2,1,0]
+    } else {
+        y = stride == 2 ? topk_dpp<0x4E>(x) : topk_dpp<0xB1>(x);  // quad_perm [2,3,0,1], [1,0,3,2]
     }
-    __syncthreads();
+    return ((x > y) == keep_min) ? y : x;
 }
 
-// `lists` independent sorted lists of width w at s + l * w: sorts each bitonic list ascending
-// (compare-exchanges at strides w/2 .. 1, all ascending).
-template <uint32_t NT>
-__device__ void topk_bitonic_merge(uint64_t* s, uint32_t lists, uint32_t w) {
-    for (uint32_t stride = w >> 1; stride > 0; stride >>= 1) {
-        __syncthreads();
-        for (uint32_t t = threadIdx.x; t < lists * (w / 2); t += NT) {
-            const uint32_t l = t / (w / 2), u = t % (w / 2);
-            const uint32_t i = l * w + 2 * u - (u & (stride - 1)), j = i + stride;
-            const uint64_t x = s[i], y = s[j];
-            if (x > y) {
-                s[i] = y;
-                s[j] = x;
-            }
-        }
+template <int V>
+struct TopkList {
+    uint64_t r[V];
+};
+
+// Sorts a bitonic list, ascending (up) or descending.
+template <int V>
+__device__ __forceinline__ void topk_merge(TopkList<V>& l, bool up) {
+    const uint32_t lane = threadIdx.x & 63u;
+    if constexpr (V == 2) {
+        const uint64_t a = l.r[0], b = l.r[1];
+        const bool swap = (a > b) == up;
+        l.r[0] = swap ? b : a;
+        l.r[1] = swap ? a : b;
     }
-    __syncthreads();
+#pragma unroll
+    for (uint32_t s = 32; s > 0; s >>= 1)
+#pragma unroll
+        for (int v = 0; v < V; ++v) l.r[v] = topk_exchange(l.r[v], s, ((lane & s) == 0) == up);
 }
 
-GH_KERNEL __launch_bounds__(512) void gh_topk_partial(GhTopkArgs a) {
-    __shared__ uint64_t s[kTopkChunk];
-    __shared__ uint64_t r[kTopkWidth];
-    const uint32_t w = a.width;
+// The smallest 64 V of an ascending and a descending list, sorted.
+template <int V>
+__device__ __forceinline__ TopkList<V> topk_least(const TopkList<V>& a, const TopkList<V>& b, bool up) {
+    TopkList<V> m;
+#pragma unroll
+    for (int v = 0; v < V; ++v) m.r[v] = min(a.r[v], b.r[v]);
+    topk_merge<V>(m, up);
+    return m;
+}
+
+// The smallest 64 V of eight vectors of 64 keys, descending.
+template <int V>
+__device__ __forceinline__ TopkList<V> topk_of_512(uint64_t (&x)[8]) {
+    const uint32_t lane = threadIdx.x & 63u;
+    // vectors 0, 2, .. ascending, 1, 3, .. descending
+#pragma unroll
+    for (uint32_t size = 2; size <= 64; size <<= 1)
+#pragma unroll
+        for (uint32_t s = size >> 1; s > 0; s >>= 1)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const bool up = ((lane & size) == 0) == ((i & 1) == 0);
+                x[i] = topk_exchange(x[i], s, ((lane & s) == 0) == up);
+            }
+    TopkList<V> l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (V == 1) {
+            l[i].r[0] = min(x[2 * i], x[2 * i + 1]);
+        } else {  // all 128 of the pair: an ascending after a descending run is bitonic
+            l[i].r[0] = x[2 * i + 1];
+            l[i].r[1] = x[2 * i];
+        }
+        topk_merge<V>(l[i], (i & 1) == 0);
+    }
+    const TopkList<V> a = topk_least<V>(l[0], l[1], true), b = topk_least<V>(l[2], l[3], false);
+    return topk_least<V>(a, b, false);
+}
+
+// One wave per stripe of a.per logits: its 64 V smallest keys, ascending, at part[stripe].
+template <int V>
+__device__ __forceinline__ void topk_partial(const GhTopkArgs& a) {
+    const uint32_t lane = threadIdx.x;
     const uint64_t b0 = (uint64_t)blockIdx.x * a.per, e = min((uint64_t)a.n, b0 + a.per);
-    const uint32_t* bits = (const uint32_t*)a.logits;
-    for (uint32_t t = threadIdx.x; t < w; t += 512) r[t] = ~0ull;
+    const GH_GLOBAL uint32_t* bits = gh_gp<uint32_t>(a.logits);
+    TopkList<V> acc;  // ascending
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc.r[v] = ~0ull;
     for (uint64_t c = b0; c < e; c += kTopkChunk) {
-        __syncthreads();
-        for (uint32_t t = threadIdx.x; t < kTopkChunk; t += 512)
-            s[t] = c + t < e ? topk_key(bits[c + t], (uint32_t)(c + t)) : ~0ull;
-        topk_sort<512>(s, kTopkChunk);
-        // the w smallest of (r, s[0, w)): r[i] = min(r[i], s[w - 1 - i]) is bitonic; sort it
-        for (uint32_t t = threadIdx.x; t < w; t += 512) r[t] = min(r[t], s[w - 1 - t]);
-        topk_bitonic_merge<512>(r, 1, w);
+        uint32_t raw[8];
+        uint64_t x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) raw[i] = bits[min(c + 64 * i + lane, e - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint64_t at = c + 64 * i + lane;
+            x[i] = at < e ? topk_key(raw[i], (uint32_t)at) : ~0ull;
+        }
+        acc = topk_least<V>(acc, topk_of_512<V>(x), true);
     }
-    for (uint32_t t = threadIdx.x; t < w; t += 512)
-        ((uint64_t*)a.part)[(size_t)blockIdx.x * w + t] = r[t];
+#pragma unroll
+    for (int v = 0; v < V; ++v) gh_gpw<uint64_t>(a.part)[((uint64_t)blockIdx.x * V + v) * 64 + lane] = acc.r[v];
+}
+GH_KERNEL __launch_bounds__(64) void gh_topk_partial(GhTopkArgs a) {
+    if (a.width == 64) topk_partial<1>(a);
+    else topk_partial<2>(a);
 }
 
-// One workgroup: the stripes' lists (padded to a power of 2 with all-ones lists) are merged
-// pairwise, halving the list count per level, keeping the w smallest keys of each pair.
+// The smallest 64 V of lists first, first + stride, ... < n at `src`, ascending: four lists at a time, the
+// odd ones read backwards.
+template <int V, class P>
+__device__ __forceinline__ TopkList<V> topk_lists(const P src, uint32_t first, uint32_t stride, uint32_t n) {
+    const uint32_t lane = threadIdx.x & 63u;
+    TopkList<V> acc;  // ascending
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc.r[v] = ~0ull;
+    for (uint32_t l0 = first; l0 < n; l0 += 4 * stride) {
+        TopkList<V> l[4];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q)
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const uint32_t li = l0 + q * stride, i = 64 * v + lane;
+                const uint64_t key = src[(uint64_t)min(li, n - 1) * 64 * V + ((q & 1) ? 64 * V - 1 - i : i)];
+                l[q].r[v] = li < n ? key : ~0ull;
+            }
+        const TopkList<V> a = topk_least<V>(l[0], l[1], true), b = topk_least<V>(l[2], l[3], false);
+        acc = topk_least<V>(acc, topk_least<V>(a, b, false), true);
+    }
+    return acc;
+}
+
+// One workgroup of 16 waves merges the stripes' lists, 16 apart per wave, then one wave the 16 lists
+// left, and writes k (u32 index, f32 bits) pairs.
+template <int V>
+__device__ __forceinline__ void topk_final(const GhTopkArgs& a, uint64_t* s) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    TopkList<V> l = topk_lists<V>(gh_gp<uint64_t>(a.part), wave, 16, a.stripes);
+#pragma unroll
+    for (int v = 0; v < V; ++v) s[(wave * V + v) * 64 + lane] = l.r[v];
+    __syncthreads();
+    if (wave) return;
+    l = topk_lists<V>((const uint64_t*)s, 0, 1, 16);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const uint32_t t = 64 * v + lane, ord = ~(uint32_t)(l.r[v] >> 32);
+        if (t >= a.k) continue;
+        gh_gpw<uint32_t>(a.out)[t] = (uint32_t)l.r[v];
+        gh_gpw<uint32_t>(a.out)[a.k + t] = ord ^ ((ord >> 31) ? 0x80000000u : 0xFFFFFFFFu);
+    }
+}
 GH_KERNEL __launch_bounds__(1024) void gh_topk_final(GhTopkArgs a) {
-    __shared__ uint64_t s[kTopkStripes * kTopkWidth];
-    const uint32_t w = a.width;
-    uint32_t lists = 1;
-    while (lists < a.stripes) lists <<= 1;
-    for (uint32_t t = threadIdx.x; t < lists * w; t += 1024)
-        s[t] = t < a.stripes * w ? ((const uint64_t*)a.part)[t] : ~0ull;
-    for (uint32_t half = lists >> 1; half > 0; half >>= 1) {
-        __syncthreads();
-        // list l (< half) takes the w smallest of itself and list l + half
-        for (uint32_t t = threadIdx.x; t < half * w; t += 1024) {
-            const uint32_t l = t / w, i = t % w;
-            s[t] = min(s[t], s[(l + half) * w + (w - 1 - i)]);
-        }
-        topk_bitonic_merge<1024>(s, half, w);
-    }
-    for (uint32_t t = threadIdx.x; t < a.k; t += 1024) {
-        const uint64_t key = s[t];
-        const uint32_t ord = ~(uint32_t)(key >> 32);
-        ((uint32_t*)a.out)[t] = (uint32_t)key;
-        ((uint32_t*)a.out)[a.k + t] = ord ^ ((ord >> 31) ? 0x80000000u : 0xFFFFFFFFu);
-    }
+    __shared__ uint64_t s[16 * 128];
+    if (a.width == 64) topk_final<1>(a, s);
+    else topk_final<2>(a, s);
 }

@@ -486,6 +486,15 @@ def test_topk_device_bit_exact(hip, vocab, ks):
     hip.free_buffer(lb)
 
 
+@pytest.mark.parametrize("vocab,ks", [
+    (64, [63, 64]), (100, [64, 65, 100]), (511, [64, 128]), (512, [65]), (513, [1, 127]),  # chunk edges
+    (131072 - 511, [64]), (131073, [64, 65]),  # 256 stripes of one chunk; 129 of two
+])
+def test_topk_device_edges(hip, vocab, ks):
+    """Both list widths (64, 128) at the edges of a wave's 512-logit chunks and of the stripe count."""
+    test_topk_device_bit_exact(hip, vocab, ks)
+
+
 # ---------------------------------------------------------------- graph driver (whole model)
 def _models(hip, shape_name, seed, kv_context, prefill_rows=64):
     from graph_horizon_amd import HipModel

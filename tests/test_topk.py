@@ -61,10 +61,10 @@ def device_value_bits(key):
     return np.where(ordv >> 31 == 1, ordv ^ 0x80000000, ordv ^ 0xFFFFFFFF)
 
 
-def device_topk(bits, k, chunk=2048, max_stripes=128):
+def device_topk(bits, k, chunk=2048, max_stripes=128, width=None):
     n = bits.size
     k = min(k, n)
-    width = 1 << (k - 1).bit_length()
+    width = width or 1 << (k - 1).bit_length()
     chunks = -(-n // chunk)
     per = chunk * -(-chunks // max_stripes)
     stripes = -(-n // per)
@@ -96,3 +96,10 @@ def test_device_scheme_matches_oracle(n, k):
     bits = SPECIALS.copy() if n == 12 else _logits(rng, n, specials=n > 5)
     want = as_bits(O.topk(bits.view(np.float32), k))
     assert device_topk(bits, k) == want
+
+
+@pytest.mark.parametrize("n,k", [(5, 3), (513, 64), (3000, 65), (131073, 64), (700000, 128)])
+def test_device_scheme_of_one_wave_stripes(n, k):
+    """The same with the kernels' sizes: 512 logits a chunk, 256 stripes, lists of 64 or 128 keys."""
+    bits = _logits(np.random.default_rng(n * 3 + k), n, specials=n > 5)
+    assert device_topk(bits, k, 512, 256, 64 if k <= 64 else 128) == as_bits(O.topk(bits.view(np.float32), k))
