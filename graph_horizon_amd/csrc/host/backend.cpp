@@ -75,6 +75,8 @@ const KernelName kKernels[] = {
     {K_GEMM3_SWIGLU_R96_T128, "gh_gemm3_swiglu_r96_t128"}, {K_GEMM3_SWIGLU_R128_T128, "gh_gemm3_swiglu_r128_t128"},
     {K_GEMM3_SWIGLU_R96, "gh_gemm3_swiglu_r96"},           {K_GEMM4W_SWIGLU_R96, "gh_gemm4w_swiglu_r96"},
     {K_GEMM3_SWIGLU_R128, "gh_gemm3_swiglu_r128"},         {K_GEMM4W_SWIGLU_R128, "gh_gemm4w_swiglu_r128"},
+    {K_GEMM5_SWIGLU, "gh_gemm5_swiglu"}, {K_GEMM5_Q4K, "gh_gemm5_q4k"}, {K_GEMM5_Q6K, "gh_gemm5_q6k"},
+    {K_GEMM5_MIXED, "gh_gemm5_mixed"},
     {K_GEMM_FEW_Q4K_T8, "gh_gemm_few_q4k_t8"}, {K_GEMM_FEW_Q6K_T8, "gh_gemm_few_q6k_t8"},
     {K_GEMM_FEW_MIXED_T8, "gh_gemm_few_mixed_t8"},
     {K_GEMM_FEW_Q4K_T16, "gh_gemm_few_q4k_t16"}, {K_GEMM_FEW_Q6K_T16, "gh_gemm_few_q6k_t16"},
@@ -1079,6 +1081,14 @@ static uint32_t gemm_block(GhKernel k) {
     }
 }
 
+// Whether `tiles` tiles of 256 rows (gh_gemm5_*) beat `small` tiles of `br` rows (gh_gemm4w_*) of an
+// unsplit launch over FP16 copies. One workgroup per CU either way, so a launch takes its tiles
+// over the CUs, rounded up, in rounds; a round of 256 rows measured 1.69 (gate and up, 8B at 2048),
+// 1.78 (14B at 500) and 1.80 (Q/K/V, 8B at 2048) rounds of 128 rows.
+static bool wide_tiles(const gh_backend* b, uint64_t tiles, uint64_t small, uint32_t br) {
+    return 9 * 128 * ceil_div(tiles, (uint64_t)b->cus) <= 5 * br * ceil_div(small, (uint64_t)b->cus);
+}
+
 static GemmPlan plan_gemm(gh_backend* b, const gh_buf* w, uint32_t n) {
     const uint32_t rows = w->rows, units = w->cols / 64;
     if (n <= kGemmFewMax) {
@@ -1127,6 +1137,8 @@ static GemmPlan plan_gemm(gh_backend* b, const gh_buf* w, uint32_t n) {
         if (s == splits) break;
         splits = s;
     }
+    if (w16 && splits == 1 && wide_tiles(b, (uint64_t)ceil_div(rows, 256) * tt, tiles, br))
+        return GemmPlan{q4 ? K_GEMM5_Q4K : K_GEMM5_Q6K, ceil_div(rows, 256), tt, 1, w16};
     return GemmPlan{k, tr, tt, splits, w16};
 }
 
@@ -1254,7 +1266,7 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
     // pairs where the separate launches take 128 rows measured 34.6 -> 36.4 ms at 2048)
     const GemmPlan pg = plan_gemm(b, wg, n), pu = plan_gemm(b, wu, n);
     const bool r96 = pg.k == K_GEMM4W_Q4K_R96 || pg.k == K_GEMM3_Q4K_R96;
-    const bool r128 = pg.k == K_GEMM4W_Q4K_R128 || pg.k == K_GEMM3_Q4K_R128;
+    const bool r128 = pg.k == K_GEMM4W_Q4K_R128 || pg.k == K_GEMM3_Q4K_R128 || pg.k == K_GEMM5_Q4K;
     // Where the separate launches split K (8B at 129-255 tokens: 128 tiles x 2 splits and a
     // split reduce), 96-row pairs unsplit instead when they fill the CUs in one pass, at least
     // half of them: the 128-token tiles' trade, in 256-token tiles
@@ -1275,6 +1287,10 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
         ga.n = n;
         ga.splits = 1;
         const bool p96t = split_pairs ? fits96 : r96;
+        // 256-row pairs (128 + 128) over the copies by the separate launches' rule
+        const uint32_t p256 = ceil_div(wg->rows, 128u);
+        if (copies && !split_pairs && wide_tiles(b, (uint64_t)p256 * tt, r96 ? p96 : p128, r96 ? 96 : 128))
+            return launch(b, K_GEMM5_SWIGLU, p256, tt, 1, 512, &ga);
         const GhKernel k = p96t ? (copies ? K_GEMM4W_SWIGLU_R96 : K_GEMM3_SWIGLU_R96)
                                 : (copies ? K_GEMM4W_SWIGLU_R128 : K_GEMM3_SWIGLU_R128);
         return launch(b, k, ceil_div(wg->rows, p96t ? 48u : 64u), tt, 1, copies ? 512 : 768, &ga);
@@ -1400,7 +1416,17 @@ int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint3
         if (rc) return rc;
         ga.part = (uint64_t)((char*)b->ws + kArgmaxBytes);
     }
-    const GhKernel k = copies ? K_GEMM4W_MIXED_R128 : tall ? K_GEMM3_MIXED_R128 : K_GEMM3_MIXED_R128_T128;
+    GhKernel k = copies ? K_GEMM4W_MIXED_R128 : tall ? K_GEMM3_MIXED_R128 : K_GEMM3_MIXED_R128_T128;
+    uint32_t wide = 0;
+    for (uint32_t i = 0; i < nseg; ++i) wide += ceil_div(segs[i].w->rows, 2 * BR);
+    if (copies && splits == 1 && wide_tiles(b, (uint64_t)wide * tt, (uint64_t)tiles * tt, BR)) {
+        k = K_GEMM5_MIXED;
+        tiles = 0;
+        for (uint32_t i = 0; i < nseg; ++i) {
+            ga.seg[i].tile0 = tiles;
+            tiles += ceil_div(segs[i].w->rows, 2 * BR);
+        }
+    }
     int rc = few ? launch_few(b, fp, ga, tiles) : launch(b, k, tiles, tt, splits, gemm_block(k), &ga);
     if (rc) return rc;
     if (splits > 1) {

@@ -126,6 +126,11 @@ enum GhKernel : int {
     K_GEMM_FEW_Q4K_T48,
     K_GEMM_FEW_Q6K_T48,
     K_GEMM_FEW_MIXED_T48,
+    // 256-row tiles over FP16 weight copies
+    K_GEMM5_SWIGLU,
+    K_GEMM5_Q4K,
+    K_GEMM5_Q6K,
+    K_GEMM5_MIXED,
     K_COUNT
 };
 

@@ -18,7 +18,8 @@
 //     one FP16 ulp when that FP32 value lands exactly on an FP16 tie.
 //   gemm4_body (over FP16 weight copies made by dequant_f16, the same values): every wave runs
 //     the matrix cores; activation lines and weight rows both arrive by LDS DMA, and the k
-//     order of every sum is gemm3_body's, so the bits are the same.
+//     order of every sum is gemm3_body's, so the bits are the same. gemm5_body is the same over
+//     256 rows, for unsplit launches whose tiles leave few rounds of the chip empty.
 // A multi-matrix launch (gemm3_mixed, the prefill's Q/K/V) runs each row tile in its matrix's
 // format over the shared LDS block. SwiGLU's gate and up run as one launch of pair tiles
 // (gh_gemm3/4w_swiglu_*): each tile holds matching gate and up rows (pair_row), K unsplit, and
@@ -682,6 +683,131 @@ GH_KERNEL __launch_bounds__(512) void gh_gemm4w_swiglu_r96(GhGemmArgs a) {
 GH_KERNEL __launch_bounds__(512) void gh_gemm4w_swiglu_r128(GhGemmArgs a) {
     __shared__ __attribute__((aligned(16))) _Float16 lds[GH_GEMM4_LDS(128)];
     gemm4_body<kQ4K, 128, true>(a, lds, blockIdx.x, blockIdx.y, blockIdx.z, a.rows, 0);
+}
+
+// The same over 256 tokens x 256 rows, K unsplit: wave w takes the 128 tokens of group w / 4
+// against rows 64 (w % 4) .. + 64 (4 x 2 tiles). gemm4_body's 64 x 64 waves are held by LDS: 176 KiB
+// of fragment reads and DMA writes (1408 cycles at 128 B each) under 1024 cycles of matrix work a
+// unit; here it is 256 KiB under 2048, and a unit brings 64 KiB from L2 for twice the work of
+// 48. Two LDS stages: the barrier of unit u stands before its last k-step's matrix work, when
+// every fragment of the unit has been read, so that unit u + 2's DMA and the first fragments
+// of unit u + 1 go out under it. The k order of every sum is gemm4_body's. What bounds it now: the DMA
+// (without it 1.25 us a unit against 1.9; the matrix work alone is 0.85), and SiLU in the
+// epilogue, which nothing overlaps. A ring of five 32-k stages, four in flight, was slower
+// (64-byte pieces of lines), as were four waves of 128 x 128 (one wave per SIMD). Gate and up of 8B at 2048 tokens
+// 462 -> 390 us, Q/K/V 157 -> 141; gate and up of 14B at 500 tokens 210 -> 186.
+constexpr uint32_t kG5Stage = 512 * 64;  // halves: 256 token rows, then 256 weight rows
+template <uint32_t FMT, bool PAIR = false>
+__device__ __forceinline__ void gemm5_body(const GhGemmArgs& a, _Float16* lds, uint32_t bx, uint32_t by) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, tg = wave >> 2, rg = wave & 3u;
+    const uint32_t r0 = bx * (PAIR ? 128 : 256), t0 = by * 256, units = a.in_dim / 64;
+    const uint32_t fm = lane & 31u, fg = lane >> 5;
+    // this wave's loads: rows 32 w + 8 i + lane / 8 of each operand, chunk (lane % 8) ^ sw(row); the
+    // activations' as byte offsets from the tile's first row (256 rows of at most 2^16 values)
+    const uint64_t xb = a.x + (uint64_t)t0 * a.in_dim * 2;
+    uint32_t xo[4];
+    uint64_t wa[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t r = 32 * wave + 8 * i + (lane >> 3), c = (lane & 7u) ^ ((r >> 1) & 7u);
+        xo[i] = min(r, a.n - 1 - t0) * a.in_dim * 2 + 2 * chunk_k<FMT>(0, c);
+        uint64_t wbase = a.w;
+        const uint32_t wr = PAIR ? pair_row<128>(r, wbase, a) : r;  // rows alternate by 32
+        wa[i] = wbase + ((uint64_t)min(r0 + wr, a.rows - 1) * units) * 128 + c * 16;
+    }
+    auto issue = [&](uint32_t u) __attribute__((always_inline)) {
+        _Float16* sa = lds + (u & 1u) * kG5Stage + 32 * wave * 64;
+        const uint64_t xu = xb + 2ull * chunk_k<FMT>(u, 0);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t da = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(sa + 8 * i * 64);
+            const uint32_t db = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(sa + (256 + 8 * i) * 64);
+            asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(xo[i]), "s"(xu),
+                         "{m0}"(__builtin_amdgcn_readfirstlane(da))
+                         : "memory");
+            asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(wa[i] + (uint64_t)u * 128),
+                         "{m0}"(__builtin_amdgcn_readfirstlane(db))
+                         : "memory");
+        }
+    };
+    f16v acc[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i][0] = acc[i][1] = f16v{};
+    struct Frags {
+        h8 a[4], b[2];
+    };
+    // k-step ks of unit u: row 32 i + fm's chunk 2 ks + fg, at slot c ^ (fm / 2) % 8
+    auto read = [&](uint32_t u, int ks, Frags& f) __attribute__((always_inline)) {
+        const _Float16* base = lds + (u & 1u) * kG5Stage + fm * 64 + ((2 * ks + fg) ^ ((fm >> 1) & 7u)) * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) f.a[i] = *(const h8*)(base + (128 * tg + 32 * i) * 64);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) f.b[j] = *(const h8*)(base + (256 + 64 * rg + 32 * j) * 64);
+    };
+    // the matrix work of f, with the next fragments' six reads spread over its eight instructions
+    auto mma = [&](const Frags& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    issue(0);
+    issue(1);  // in_dim is a multiple of 256: at least four units
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // unit 0's part of this wave has landed
+    __syncthreads();
+    Frags f0, f1;
+    read(0, 0, f0);
+    for (uint32_t u = 0; u < units; ++u) {
+        read(u, 1, f1);
+        mma(f0);
+        read(u, 2, f0);
+        mma(f1);
+        read(u, 3, f1);
+        mma(f0);
+        // this wave's part of unit u + 1 has landed and its reads of unit u are done
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (u + 2 < units) issue(u + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        read(u + 1 < units ? u + 1 : u, 0, f0);  // the last one reads landed data nobody uses
+        mma(f1);
+    }
+    if constexpr (PAIR) pair_write128(a, acc, t0 + 128 * tg, r0 + 32 * rg, fm, fg);
+    else gemm_write<4, 2, true>(a, acc, t0 + 128 * tg, r0 + 64 * rg, fm, fg, 0, a.rows, 0);
+}
+GH_KERNEL __launch_bounds__(512) void gh_gemm5_swiglu(GhGemmArgs a) {
+    __shared__ __attribute__((aligned(16))) _Float16 lds[2 * kG5Stage];
+    gemm5_body<kQ4K, true>(a, lds, blockIdx.x, blockIdx.y);
+}
+GH_KERNEL __launch_bounds__(512) void gh_gemm5_q4k(GhGemmArgs a) {
+    __shared__ __attribute__((aligned(16))) _Float16 lds[2 * kG5Stage];
+    gemm5_body<kQ4K>(a, lds, blockIdx.x, blockIdx.y);
+}
+GH_KERNEL __launch_bounds__(512) void gh_gemm5_q6k(GhGemmArgs a) {
+    __shared__ __attribute__((aligned(16))) _Float16 lds[2 * kG5Stage];
+    gemm5_body<kQ6K>(a, lds, blockIdx.x, blockIdx.y);
+}
+// several matrices (a.seg, row tiles of 256)
+GH_KERNEL __launch_bounds__(512) void gh_gemm5_mixed(GhGemmArgs a) {
+    __shared__ __attribute__((aligned(16))) _Float16 lds[2 * kG5Stage];
+    uint32_t s = 0;
+    for (uint32_t i = 1; i < a.nseg; ++i)
+        if (blockIdx.x >= a.seg[i].tile0) s = i;
+    GhGemmArgs m = a;
+    m.w = a.seg[s].w;
+    m.rows = a.seg[s].rows;
+    m.out = a.seg[s].out;
+    const uint32_t bx = blockIdx.x - a.seg[s].tile0;
+    if (a.seg[s].fmt == kQ4K) gemm5_body<kQ4K>(m, lds, bx, blockIdx.y);
+    else gemm5_body<kQ6K>(m, lds, bx, blockIdx.y);
 }
 
 // A Q4_K / Q6_K matrix [rows][in_dim] dequantized to FP16 in the GEMM's unit order, the layout

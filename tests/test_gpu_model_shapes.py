@@ -183,6 +183,34 @@ def test_prefill_fp16_weight_copies_are_bit_identical(hip, name, n):
         assert np.array_equal(got, want), what
 
 
+@pytest.mark.parametrize("name,n,heads", [("8b", 1793, (32, 8)), ("14b", 2047, (32, 8)), ("14b", 257, (32, 8)),
+                                          ("8b", 2000, (40, 5))])
+def test_prefill_256_row_tiles_are_bit_identical(hip, name, n, heads):
+    """Long prefills over the FP16 copies in tiles of 256 rows (gh_gemm5_*) against the dequantizing
+    kernels: the same k order, so the same bits. One token in the last tile, one missing, a second tile
+    of one token (gate and up alone take the 256-row tiles), and K and V of 640 rows, whose
+    last row tile is half full."""
+    from graph_horizon_amd import _ffi as F
+
+    shape = dataclasses.replace(synth.SHAPES[name], name=f"{name}-wide", block_count=1, head_count=heads[0],
+                                kv_head_count=heads[1])
+    seed = 23
+    tensors = list(synth.model_tensors(shape, seed))
+    toks = [int(t) for t in np.random.default_rng(seed).integers(0, shape.vocab_size, n)]
+    outs = []
+    for flags in (0, F.MODEL_NO_F16_WEIGHTS):
+        gm = HipModel(hip, synth.model_config(shape, n, prefill_rows=n, flags=flags))
+        for layer, tid, fmt, data in tensors:
+            gm.load_tensor(layer, tid, fmt, data)
+        gm.prefill(toks, 0)
+        kv, m = gm.kv(), n * shape.kv_head_count * shape.head_dim
+        outs.append((gm.read_logits().view(np.uint32), gm.read_x().view(np.uint32),
+                     hip.download(kv.k, np.uint16, m), hip.download(kv.v, np.uint16, m)))
+        gm.close()
+    for got, want, what in zip(outs[0], outs[1], ("logits", "x", "k", "v")):
+        assert np.array_equal(got, want), what
+
+
 def test_prefill_fp16_weight_copies_follow_reloaded_weights(hip):
     """The FP16 copies are a cache of the layer matrices: reloading a matrix after a prefill
     made them (gh_model_load_tensor) drops every copy, and the next prefill dequantizes the new
