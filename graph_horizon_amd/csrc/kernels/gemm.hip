@@ -151,9 +151,33 @@ __device__ __forceinline__ void store_w(uint32_t u, const WStage& ws, _Float16* 
                                         uint32_t tid = threadIdx.x) {
     const uint32_t row = tid % BR, part = tid / BR;
     _Float16* dst = wb + row * LDK;
+    const uint32_t qw[4] = {ws.q.x, ws.q.y, ws.q.z, ws.q.w};
     uint32_t lo[8], hi[8];
-    if constexpr (FMT == kQ4K) gh_w16_q4k(ws.q, ws.hd, u & 3u, lo, hi);
-    else gh_w16_q6k(ws.q, ws.qh, ws.hd, ws.d, (u >> 1) & 1u, u & 1u, part, lo, hi);
+    if constexpr (FMT == kQ4K) {
+        const GhW16Q4K c = gh_w16_q4k_scales(ws.hd, u & 3u);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t lo4 = qw[j] & 0x0F0F0F0Fu, hi4 = (qw[j] >> 4) & 0x0F0F0F0Fu;
+            // opaque: with the masks' known zero bits the compiler would extract each byte
+            // separately instead of converting it in place (v_cvt_f32_ubyte1..3)
+            asm volatile("" : "+v"(lo4), "+v"(hi4));
+            lo[2 * j] = gh_w16_q4k_pair(lo4, 0, c.d1, c.m1);
+            lo[2 * j + 1] = gh_w16_q4k_pair(lo4, 2, c.d1, c.m1);
+            hi[2 * j] = gh_w16_q4k_pair(hi4, 0, c.d2, c.m2);
+            hi[2 * j + 1] = gh_w16_q4k_pair(hi4, 2, c.d2, c.m2);
+        }
+    } else {
+        const GhW16Q6K c = gh_w16_q6k_scales(ws.hd, ws.d, (u >> 1) & 1u, u & 1u, part);
+        const uint32_t qh[4] = {ws.qh.x, ws.qh.y, ws.qh.z, ws.qh.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t qa4 = gh_w16_q6k_low(qw[j], qh[j], part), qb4 = gh_w16_q6k_high(qw[j], qh[j], part);
+            lo[2 * j] = gh_w16_q6k_pair(qa4, 0, c.da, c.na);
+            lo[2 * j + 1] = gh_w16_q6k_pair(qa4, 2, c.da, c.na);
+            hi[2 * j] = gh_w16_q6k_pair(qb4, 0, c.db, c.nb);
+            hi[2 * j + 1] = gh_w16_q6k_pair(qb4, 2, c.db, c.nb);
+        }
+    }
     // low nibbles (quarter 2·part for Q6_K): positions 16·part + i; high: 32 + 16·part + i
     *(uint4*)(dst + 16 * part) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
     *(uint4*)(dst + 16 * part + 8) = make_uint4(lo[4], lo[5], lo[6], lo[7]);

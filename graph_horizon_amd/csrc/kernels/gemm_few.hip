@@ -111,6 +111,35 @@ __device__ __forceinline__ uint32_t lane_k(uint32_t u) {
     return FMT == kQ4K ? 64 * u : 128 * (u >> 1) + 16 * (u & 1u);
 }
 
+// 32 FP16-rounded weights of a unit: lo = the low nibbles of 16 quant bytes, hi = the high ones, as
+// natural-order pairs. Q4_K: q = half of the group's qs bytes; Q6_K: q = 16 bytes of ql plane `part`.
+__device__ __forceinline__ void w16_q4k(const uint4& q, const uint4& hd, uint32_t g, uint32_t (&lo)[8], uint32_t (&hi)[8]) {
+    const GhW16Q4K c = gh_w16_q4k_scales(hd, g);
+    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        uint32_t lo4 = qw[j] & 0x0F0F0F0Fu, hi4 = (qw[j] >> 4) & 0x0F0F0F0Fu;
+        asm volatile("" : "+v"(lo4), "+v"(hi4));  // bytes converted in place, as in the tiles' store_w
+        lo[2 * j] = gh_w16_q4k_pair(lo4, 0, c.d1, c.m1);
+        lo[2 * j + 1] = gh_w16_q4k_pair(lo4, 2, c.d1, c.m1);
+        hi[2 * j] = gh_w16_q4k_pair(hi4, 0, c.d2, c.m2);
+        hi[2 * j + 1] = gh_w16_q4k_pair(hi4, 2, c.d2, c.m2);
+    }
+}
+__device__ __forceinline__ void w16_q6k(const uint4& q, const uint4& qhv, const uint2& sc, uint32_t dh, uint32_t part,
+                                        uint32_t (&lo)[8], uint32_t (&hi)[8]) {
+    const GhW16Q6K c = gh_w16_q6k_scales(make_uint4(sc.x, sc.y, 0u, 0u), dh, 0, 0, part);
+    const uint32_t qw[4] = {q.x, q.y, q.z, q.w}, qh[4] = {qhv.x, qhv.y, qhv.z, qhv.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t qa4 = gh_w16_q6k_low(qw[j], qh[j], part), qb4 = gh_w16_q6k_high(qw[j], qh[j], part);
+        lo[2 * j] = gh_w16_q6k_pair(qa4, 0, c.da, c.na);
+        lo[2 * j + 1] = gh_w16_q6k_pair(qa4, 2, c.da, c.na);
+        hi[2 * j] = gh_w16_q6k_pair(qb4, 0, c.db, c.nb);
+        hi[2 * j + 1] = gh_w16_q6k_pair(qb4, 2, c.db, c.nb);
+    }
+}
+
 // Two row tiles x NT token tiles of 16: acc += x · (B fragments of 16 weights, k offset `ko` halves
 // from the lane's first), chunk by chunk.
 template <int NT>
@@ -142,7 +171,7 @@ __device__ __forceinline__ void block_w16(const Unit<FMT> (&w)[2], const Staged&
     for (int h = 0; h < 2; ++h) {
         if constexpr (FMT == kQ4K) {
 #pragma unroll
-            for (int r = 0; r < 2; ++r) gh_w16_q4k(w[r].q[h], w[r].hd, u, lo[r], hi[r]);
+            for (int r = 0; r < 2; ++r) w16_q4k(w[r].q[h], w[r].hd, u, lo[r], hi[r]);
             mma16<NT>(xr, 16 * h, lo[0], lo[1], acc);
             mma16<NT>(xr, 32 + 16 * h, hi[0], hi[1], acc);
             __builtin_amdgcn_sched_barrier(0);  // one half's fragments live at a time
@@ -150,7 +179,7 @@ __device__ __forceinline__ void block_w16(const Unit<FMT> (&w)[2], const Staged&
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 const uint2 sc = q6_scales(w[r].sc, u);
-                gh_w16_q6k(h ? w[r].b : w[r].a, w[r].h, make_uint4(sc.x, sc.y, 0u, 0u), w[r].d, 0, 0, h, lo[r], hi[r]);
+                w16_q6k(h ? w[r].b : w[r].a, w[r].h, sc, w[r].d, h, lo[r], hi[r]);
             }
             mma16<NT>(xr, 32 * h, lo[0], lo[1], acc);
             mma16<NT>(xr, 64 + 32 * h, hi[0], hi[1], acc);

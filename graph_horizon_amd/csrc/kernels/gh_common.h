@@ -142,84 +142,68 @@ __device__ __forceinline__ void gh_q4k_scale_min(const uint4& hd, uint32_t j, ui
     mn = ((zs & 63u) & ~hi) | ((((ws >> 4) & 15u) | ((zs >> 2) & 48u)) & hi);
 }
 
-// FP16 weights of the prefill GEMMs, 32 at a time: lo = the low nibbles of 16 quant bytes, hi = the
-// high ones, as natural-order FP16 pairs.
-// Q4_K: q = 16 qs bytes of group g (sub-blocks 2 g and 2 g + 1), hd = the block header.
-__device__ __forceinline__ void gh_w16_q4k(const uint4& q, const uint4& hd, uint32_t g, uint32_t (&lo)[8],
-                                   uint32_t (&hi)[8]) {
-#pragma clang fp contract(off)
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+// FP16 weights of the prefill GEMMs, a block's quants two at a time. (Whole units behind one function,
+// its 16 dwords returned through references, cost the tiles 128 wait states a unit: 128 x 4096 ->
+// 2 x 12288 45.0 instead of 44.4 us.)
+// Q4_K: the scale and minimum of sub-blocks 2 g (low nibbles of a group) and 2 g + 1 (high ones).
+// d·sc and dmin·mn are exact in FP32 (an FP16 times a 6-bit integer), and so is (d·sc)·q for a 4-bit
+// q (at most 21 significant bits): the reference's product, then difference, rounds once, as one FMA
+// does, so the FMA gives the same FP32 value.
+struct GhW16Q4K {
+    float d1, m1, d2, m2;
+};
+__device__ __forceinline__ GhW16Q4K gh_w16_q4k_scales(const uint4& hd, uint32_t g) {
     uint32_t sc0, mn0, sc1, mn1;
     gh_q4k_scale_min(hd, 2 * g, sc0, mn0);
     gh_q4k_scale_min(hd, 2 * g + 1, sc1, mn1);
     const float d = gh_h2f(hd.x & 0xFFFFu), dmin = gh_h2f(hd.x >> 16);
-    const float d1 = d * (float)sc0, m1 = dmin * (float)mn0;
-    const float d2 = d * (float)sc1, m2 = dmin * (float)mn1;
-    // nibbles four at a time: byte e of lo4 / hi4 is the low / high nibble of byte e.
-    // d·sc and dmin·mn are exact in FP32 (an FP16 times a 6-bit integer), and so is
-    // (d·sc)·q for a 4-bit q (at most 21 significant bits): the reference's product,
-    // then difference, rounds once, as one FMA does, so the FMA gives the same FP32 value.
-    auto w2 = [](uint32_t q4, int e, float sc, float mn) __attribute__((always_inline)) {
-        typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
-        const float f0 = (float)((q4 >> (8 * e)) & 0xFFu), f1 = (float)((q4 >> (8 * e + 8)) & 0xFFu);
-        float v0 = __builtin_fmaf(sc, f0, -mn), v1 = __builtin_fmaf(sc, f1, -mn);
-        // the FP32 values are rounded to FP16 as a second step (v_cvt_pk_f16_f32), not fused
-        // into one rounding of the exact value (v_fma_mix), which differs on FP16 ties
-        asm volatile("" : "+v"(v0), "+v"(v1));
-        const hv2 r = {(_Float16)v0, (_Float16)v1};
-        return __builtin_bit_cast(uint32_t, r);
-    };
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        uint32_t lo4 = qw[j] & 0x0F0F0F0Fu, hi4 = (qw[j] >> 4) & 0x0F0F0F0Fu;
-        // opaque: with the masks' known zero bits the compiler would extract each byte
-        // separately instead of converting it in place (v_cvt_f32_ubyte1..3)
-        asm volatile("" : "+v"(lo4), "+v"(hi4));
-        lo[2 * j] = w2(lo4, 0, d1, m1);
-        lo[2 * j + 1] = w2(lo4, 2, d1, m1);
-        hi[2 * j] = w2(hi4, 0, d2, m2);
-        hi[2 * j + 1] = w2(hi4, 2, d2, m2);
-    }
+    return GhW16Q4K{d * (float)sc0, dmin * (float)mn0, d * (float)sc1, dmin * (float)mn1};
+}
+// Bytes e and e + 1 of q4 (a nibble each) as weights.
+__device__ __forceinline__ uint32_t gh_w16_q4k_pair(uint32_t q4, int e, float sc, float mn) {
+#pragma clang fp contract(off)
+    typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
+    const float f0 = (float)((q4 >> (8 * e)) & 0xFFu), f1 = (float)((q4 >> (8 * e + 8)) & 0xFFu);
+    float v0 = __builtin_fmaf(sc, f0, -mn), v1 = __builtin_fmaf(sc, f1, -mn);
+    // the FP32 values are rounded to FP16 as a second step (v_cvt_pk_f16_f32), not fused
+    // into one rounding of the exact value (v_fma_mix), which differs on FP16 ties
+    asm volatile("" : "+v"(v0), "+v"(v1));
+    const hv2 r = {(_Float16)v0, (_Float16)v1};
+    return __builtin_bit_cast(uint32_t, r);
 }
 
-// Q6_K: q = 16 bytes of ql plane `part` of unit (segment s, half h), qhv = the unit's qh bytes, sc =
-// the block's int8 scales, dh = its FP16 scale.
-__device__ __forceinline__ void gh_w16_q6k(const uint4& q, const uint4& qhv, const uint4& sc, uint32_t dh, uint32_t s,
-                                   uint32_t h, uint32_t part, uint32_t (&lo)[8], uint32_t (&hi)[8]) {
-#pragma clang fp contract(off)
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
-    // part 0: ql plane a -> quarters 0 (low nibble, qh bits 0-1) and 2 (high, bits 4-5);
-    // part 1: plane b -> quarters 1 (bits 2-3) and 3 (bits 6-7). Scale of quarter q:
-    // int8 scales[8s + h + 2q]. Four quants per dword: the nibble and the two high bits
-    // are combined byte-parallel into unsigned 6-bit values u, and each weight is
-    // (u - 32)·da = u·da + (-32·da) (the bias exact: a power-of-two multiple), one fused
-    // multiply-add rounded once to FP16.
+// Q6_K: the scales of quarters `part` (low nibbles of ql plane `part`, qh bits 2 part, 2 part + 1) and
+// part + 2 (high nibbles, qh bits 4 + 2 part, 5 + 2 part) of unit (segment s, half h) and their -32-fold.
+// Scale of quarter q: int8 scales[8 s + h + 2 q]; dh = the block's FP16 scale.
+struct GhW16Q6K {
+    float da, db, na, nb;
+};
+__device__ __forceinline__ GhW16Q6K gh_w16_q6k_scales(const uint4& sc, uint32_t dh, uint32_t s, uint32_t h,
+                                                      uint32_t part) {
     const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
     const uint32_t ia = 8 * s + h + 2 * part, ib = ia + 4;
     const float d = gh_h2f(dh);
     const float da = d * (float)(int8_t)(scw[ia >> 2] >> (8 * (ia & 3u)));
     const float db = d * (float)(int8_t)(scw[ib >> 2] >> (8 * (ib & 3u)));
-    const float na = -32.0f * da, nb = -32.0f * db;
-    const uint32_t qh[4] = {qhv.x, qhv.y, qhv.z, qhv.w};
-    // the two high bits of each quant moved to bits 4-5 of its byte in one shift:
-    // ((qh >> 2 part) & 3) << 4 = (qh << (4 - 2 part)) & 0x30, ((qh >> (4 + 2 part)) & 3) << 4
-    // = (qh >> 2 part) & 0x30 (part is 0 or 1)
-    const uint32_t sl = 4 - 2 * part, sh = 2 * part;
-    auto w2 = [](uint32_t q4, int e, float sc, float bias) __attribute__((always_inline)) {
-        typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
-        const float f0 = (float)((q4 >> (8 * e)) & 0xFFu), f1 = (float)((q4 >> (8 * e + 8)) & 0xFFu);
-        const hv2 r = {(_Float16)__builtin_fmaf(f0, sc, bias), (_Float16)__builtin_fmaf(f1, sc, bias)};
-        return __builtin_bit_cast(uint32_t, r);
-    };
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t qa4 = (qw[j] & 0x0F0F0F0Fu) | ((qh[j] << sl) & 0x30303030u);
-        const uint32_t qb4 = ((qw[j] >> 4) & 0x0F0F0F0Fu) | ((qh[j] >> sh) & 0x30303030u);
-        lo[2 * j] = w2(qa4, 0, da, na);
-        lo[2 * j + 1] = w2(qa4, 2, da, na);
-        hi[2 * j] = w2(qb4, 0, db, nb);
-        hi[2 * j + 1] = w2(qb4, 2, db, nb);
-    }
+    return GhW16Q6K{da, db, -32.0f * da, -32.0f * db};
+}
+// Four quants of either quarter in a dword's bytes, unsigned: the nibbles with the two high bits moved
+// to bits 4-5 of their byte in one shift: ((qh >> 2 part) & 3) << 4 = (qh << (4 - 2 part)) & 0x30,
+// ((qh >> (4 + 2 part)) & 3) << 4 = (qh >> 2 part) & 0x30 (part is 0 or 1).
+__device__ __forceinline__ uint32_t gh_w16_q6k_low(uint32_t ql, uint32_t qh, uint32_t part) {
+    return (ql & 0x0F0F0F0Fu) | ((qh << (4 - 2 * part)) & 0x30303030u);
+}
+__device__ __forceinline__ uint32_t gh_w16_q6k_high(uint32_t ql, uint32_t qh, uint32_t part) {
+    return ((ql >> 4) & 0x0F0F0F0Fu) | ((qh >> (2 * part)) & 0x30303030u);
+}
+// Bytes e and e + 1 of q4 as weights: (u - 32)·da = u·da + (-32·da) (the bias exact: a power-of-two
+// multiple), one fused multiply-add rounded once to FP16.
+__device__ __forceinline__ uint32_t gh_w16_q6k_pair(uint32_t q4, int e, float sc, float bias) {
+#pragma clang fp contract(off)
+    typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
+    const float f0 = (float)((q4 >> (8 * e)) & 0xFFu), f1 = (float)((q4 >> (8 * e + 8)) & 0xFFu);
+    const hv2 r = {(_Float16)__builtin_fmaf(f0, sc, bias), (_Float16)__builtin_fmaf(f1, sc, bias)};
+    return __builtin_bit_cast(uint32_t, r);
 }
 
 #endif
