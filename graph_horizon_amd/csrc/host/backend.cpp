@@ -1216,11 +1216,12 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
     const uint64_t cells = (uint64_t)n * wg->rows;
     if (!fits(a, (uint64_t)n * wg->cols * 2) || !fits(out, cells * 2) || !fits(gate, cells * 2))
         return fail(b, GH_E_RANGE, "gemm swiglu: buffer too small");
-    if (n <= kGemmFewMax && wg->rows % 4 == 0) {
+    const FewPlan f = plan_few(wg->cols, std::min(n, kGemmFewMax));
+    const uint64_t few_half = (uint64_t)f.splits * cells;
+    if (n <= kGemmFewMax && wg->rows % 4 == 0 && few_half <= 0xFFFFFFFFull) {
         // few tokens: both matrices in one launch, partials [2][splits][n][rows] for the shared reduce
-        const FewPlan f = plan_few(wg->cols, n);
-        const uint64_t half = (uint64_t)f.splits * cells;
-        int rc = ensure_workspace(b, 2 * half * 4);
+        // (the second matrix's start is a 32-bit field)
+        int rc = ensure_workspace(b, 2 * few_half * 4);
         if (rc) return rc;
         GhGemmArgs ga{};
         ga.x = a->addr;
@@ -1232,7 +1233,7 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
         ga.nseg = 2;
         const uint32_t tiles = ceil_div(wg->rows, 128);
         ga.seg[0] = GhGemmSeg{wg->addr, 0, wg->rows, wg->format, 0, 0, 0, 0};
-        ga.seg[1] = GhGemmSeg{wu->addr, 0, wg->rows, wu->format, tiles, 0, 0, (uint32_t)half};
+        ga.seg[1] = GhGemmSeg{wu->addr, 0, wg->rows, wu->format, tiles, 0, 0, (uint32_t)few_half};
         rc = launch_few(b, f, ga, 2 * tiles);
         if (rc) return rc;
         ga.out = out->addr;
@@ -1477,7 +1478,12 @@ static int gemv_launch(gh_backend* b, const gh_buf* out, const gh_buf* a, const 
     // 4096 x 4096 Q4_K at 2 / 5 tokens 8.3 / 16.1 us against 9.6 / 10.2, 1024 x 4096 Q6_K 4.9 / 8.6
     // against 10.0 / 10.5, 12288 x 4096 14.9 / 32.7 against 13.3 / 13.4)
     const bool small = n < 8 && n * w->bytes <= (uint64_t)24 << 20;
-    if (!f32 && n >= kGemmMinTokens && !small) return op_gemm(b, out->addr, a, w, n);
+    if (!f32 && n >= kGemmMinTokens && !small) {
+        const int rc = op_gemm(b, out->addr, a, w, n);
+        if (rc != GH_E_OOM || n >= 8) return rc;
+        (void)hipGetLastError();  // no room for the partials: the GEMV needs none
+        b->err.clear();
+    }
     GemvSeg seg{w, out->addr, f32 ? (uint32_t)GH_EPI_F32 : (uint32_t)GH_EPI_F16};
     return op_gemv(b, &seg, 1, a, n, 0, nullptr, 0, nullptr);
 }
