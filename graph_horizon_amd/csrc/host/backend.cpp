@@ -1431,9 +1431,7 @@ int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint3
     int rc = few ? launch_few(b, fp, ga, tiles) : launch(b, k, tiles, tt, splits, gemm_block(k), &ga);
     if (rc) return rc;
     if (splits > 1) {
-        const uint64_t npairs = (uint64_t)n * total / 2;
-        return launch(b, K_GEMM_REDUCE_SEG, (uint32_t)std::min<uint64_t>(ceil_div(npairs, (uint64_t)256), 4096), 1, 1,
-                      256, &ga);
+        return launch(b, K_GEMM_REDUCE_SEG, n, ceil_div(total, 512), 1, 256, &ga);
     }
     if (nseg >= 2 && segs[0].role == GH_GEMM_ROLE_ROPE_QUERY && segs[1].role == GH_GEMM_ROLE_ROPE_KEY &&
         (nseg < 3 || !segs[2].role))
