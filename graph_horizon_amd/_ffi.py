@@ -126,6 +126,7 @@ SIGNATURES = {
     "gh_set_attention_xcd_merge": (I32, [P, I32]),
     "gh_xcd_count": (U32, [P]),
     "gh_stream_probe": (I32, [P, P, BUFP, U64, U64, BUFP, U32]),
+    "gh_set_scratch_limit": (I32, [P, U64]),
     "gh_scratch_info": (I32, [P, C.POINTER(U64), C.POINTER(U64), C.POINTER(U64)]),
     "gh_model_create": (I32, [P, C.POINTER(GhModelConfig), C.POINTER(P)]),
     "gh_model_destroy": (None, [P]),

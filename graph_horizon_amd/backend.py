@@ -221,6 +221,10 @@ class HipBackend:
                  "scratch_info")
         return ws.value, cs.value, gen.value
 
+    def set_scratch_limit(self, nbytes: int):
+        """Largest workspace (and counter block) the backend may grow to; 0 = no bound."""
+        self._ok(self.lib.gh_set_scratch_limit(self.h, nbytes), "set_scratch_limit")
+
     def set_attention_splits(self, splits: int):
         """Decode attention workgroups per (row, kv head); 0 = the backend's policy."""
         self._ok(self.lib.gh_set_attention_splits(self.h, splits), "set_attention_splits")

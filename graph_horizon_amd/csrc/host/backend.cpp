@@ -195,20 +195,52 @@ int launch(gh_backend* b, GhKernel k, uint32_t gx, uint32_t gy, uint32_t gz, uin
                      "hipModuleLaunchKernel");
 }
 
+// Moves a growable scratch block (`bytes` long, its content not kept) to one of `want` bytes. Without
+// room beside the old block, that is freed first; without room for the new one even then, the old size is
+// allocated again, so that a caller with a smaller launch to fall back on still has what it had. The
+// generation advances with every change of *block, a failed growth's too: recorded graphs hold the
+// address.
+static int regrow(gh_backend* b, void** block, size_t* bytes, size_t want, const char* what) {
+    auto alloc = [&](void** p, size_t n) {
+        return b->scratch_limit && n > b->scratch_limit ? hipErrorOutOfMemory : hipMalloc(p, n);
+    };
+    int rc = hip_check(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+    if (rc) return rc;
+    void* fresh = nullptr;
+    hipError_t e = alloc(&fresh, want);
+    if (e == hipSuccess && *block) (void)hipFree(*block);
+    if (e == hipErrorOutOfMemory && *block) {
+        const size_t had = *bytes;
+        (void)hipFree(*block);
+        *block = nullptr;
+        *bytes = 0;
+        ++b->gen;
+        e = alloc(&fresh, want);
+        if (e != hipSuccess && alloc(block, had) == hipSuccess) *bytes = had;
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next check in the process
+        return hip_check(b, e, what);
+    }
+    *block = fresh;
+    *bytes = want;
+    ++b->gen;
+    return GH_OK;
+}
+
 int ensure_workspace(gh_backend* b, size_t bytes) {
     bytes += kArgmaxBytes;
     if (b->ws_bytes >= bytes) return GH_OK;
     if (b->capturing) return fail(b, GH_E_STATE, "workspace growth during graph capture");
-    int rc = hip_check(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-    if (rc) return rc;
-    if (b->ws) (void)hipFree(b->ws);
-    b->ws = nullptr;
-    b->ws_bytes = 0;
-    size_t want = std::max(bytes, (size_t)(4u << 20));
-    rc = hip_check(b, hipMalloc(&b->ws, want), "hipMalloc(workspace)");
-    if (rc) return rc;
-    b->ws_bytes = want;
-    ++b->gen;
+    return regrow(b, &b->ws, &b->ws_bytes, std::max(bytes, (size_t)(4u << 20)), "hipMalloc(workspace)");
+}
+
+// Workspace for a launch that has a form with less: *room = false, and no error, where it cannot be had.
+static int try_workspace(gh_backend* b, size_t bytes, bool* room) {
+    const int rc = ensure_workspace(b, bytes);
+    *room = rc == GH_OK;
+    if (rc != GH_E_OOM) return rc;
+    b->err.clear();
     return GH_OK;
 }
 
@@ -329,18 +361,14 @@ int ensure_counters(gh_backend* b, size_t slots) {
     if (b->counter_slots >= slots) return GH_OK;
     if (b->capturing) return fail(b, GH_E_STATE, "counter growth during graph capture");
     slots = std::max<size_t>(slots, 4096);
-    int rc = hip_check(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-    if (rc) return rc;
-    if (b->counters) (void)hipFree(b->counters);
-    b->counters = nullptr;
+    size_t bytes = b->counter_slots * 4;
+    const int rc = regrow(b, &b->counters, &bytes, slots * 4, "hipMalloc(counters)");
     b->counter_slots = 0;
-    rc = hip_check(b, hipMalloc(&b->counters, slots * 4), "hipMalloc(counters)");
-    // on the (non-blocking) backend stream, so the clear is ordered before every launch
-    if (!rc) rc = hip_check(b, hipMemsetAsync(b->counters, 0, slots * 4, b->stream), "hipMemsetAsync(counters)");
-    if (rc) return rc;
-    b->counter_slots = slots;
-    ++b->gen;
-    return GH_OK;
+    // cleared (also those of the old size after a failed growth) on the (non-blocking) backend stream,
+    // ordered before every launch
+    const int rz = bytes ? hip_check(b, hipMemsetAsync(b->counters, 0, bytes, b->stream), "hipMemsetAsync(counters)") : GH_OK;
+    if (!rz) b->counter_slots = bytes / 4;
+    return rc ? rc : rz;
 }
 
 // Key splits of a prefill attention launch of `wgs` 16-row workgroups whose longest query block
@@ -375,14 +403,10 @@ static int attention_prefill(gh_backend* b, GhAttnArgs a, uint32_t group) {
     uint32_t splits = prefill_splits(b, nqb * ng, ceil_div(a.base + a.rows, 64));
     if (splits > 1) {
         const size_t n = (size_t)a.rows * a.q_heads * splits;
-        const int rc = ensure_workspace(b, attention_workspace(a.rows, a.q_heads, splits));
-        if (rc == GH_E_OOM) {  // no room for the partials: one split
-            (void)hipGetLastError();
-            b->err.clear();
-            splits = 1;
-        } else if (rc) {
-            return rc;
-        }
+        bool room = false;
+        const int rc = try_workspace(b, attention_workspace(a.rows, a.q_heads, splits), &room);
+        if (rc) return rc;
+        if (!room) splits = 1;
         char* ws = (char*)b->ws + kArgmaxBytes;
         a.part_m = (uint64_t)ws;
         a.part_l = (uint64_t)(ws + n * 4);
@@ -1714,6 +1738,12 @@ int gh_stream_probe(gh_backend* b, gh_encoder* enc, const gh_buf* src, uint64_t 
         return latch(enc, fail(b, GH_E_RANGE, "stream probe: beyond buffer"));
     GhEltArgs e{sink->addr, src->addr + offset, 0, (uint32_t)(bytes / 16), workgroups};
     return latch(enc, launch(b, K_STREAM_PROBE, workgroups, 1, 1, 256, &e));
+}
+
+int gh_set_scratch_limit(gh_backend* b, uint64_t bytes) {
+    if (!b) return GH_E_INVALID;
+    b->scratch_limit = bytes;
+    return GH_OK;
 }
 
 int gh_scratch_info(const gh_backend* b, uint64_t* workspace_bytes, uint64_t* counter_slots,

@@ -168,6 +168,7 @@ struct gh_backend {
     size_t ws_bytes = 0;
     void* counters = nullptr;  // attention merge counters, zero between launches
     size_t counter_slots = 0;
+    size_t scratch_limit = 0;  // gh_set_scratch_limit: larger scratch blocks fail as without memory; 0: none
     GhRopeTable rope;  // the trait ops' table (gh_rope_yarn, gh_rope_yarn_batched)
     uint32_t attn_splits = 0;  // gh_set_attention_splits: 0 = attention_splits' policy
     // XCDs of the device when its dispatcher was seen to place workgroup i of every probed

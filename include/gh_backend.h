@@ -236,6 +236,12 @@ int gh_stream_probe(gh_backend* b, gh_encoder* enc, const gh_buf* src, uint64_t 
 int gh_scratch_info(const gh_backend* b, uint64_t* workspace_bytes, uint64_t* counter_slots,
                     uint64_t* generation);
 
+/* Bounds each growable scratch block (workspace, merge counters) of the backend to `bytes`, 0 = no
+ * bound (no counterpart in the reference: a test hook). A growth past it fails as hipMalloc does without
+ * memory: launches with a form that needs less take that, others return GH_E_OOM. What is allocated
+ * stays. */
+int gh_set_scratch_limit(gh_backend* b, uint64_t bytes);
+
 /* =====================================================================================
  * Graph driver: a C++ restatement of the caller side of the boundary — MistralGraph's pinned
  * op order for one token (family/mistral/graph/forward.rs:68-83, block.rs:17-107,

@@ -256,6 +256,49 @@ def test_greedy_graph_with_forced_splits_matches_stream(hip):
     assert np.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("kept", [True, False], ids=["old-size-kept", "nothing-kept"])
+def test_failed_scratch_growth_re_records_decode_graphs(kept):
+    """A prefill attention launch whose partials do not fit runs unsplit. The failed growth may have
+    moved or given up the workspace that recorded decode graphs write, so they are recorded again (or,
+    without any workspace, the decode reports it) instead of replayed over freed memory."""
+    from graph_horizon_amd import GhError, HipBackend, HipModel, synth
+
+    shape, rng = synth.SHAPES["tiny"], np.random.default_rng(6)
+    n, base, qh, kvh = 100, 4000, 32, 8  # six key splits: 10 MB of partials
+    ctx = base + n
+    kc, vc = (O.f16(rng.standard_normal(ctx * kvh * 128).astype(np.float32)) for _ in range(2))
+    q = O.f16(rng.standard_normal(n * qh * 128).astype(np.float32))
+    want = O.f32(O.attention_prefill(q, kc, vc, 128, kvh, qh, base, n, 0, ctx))
+    with HipBackend(0) as b:
+        kv = _kv(b, 1, ctx, kvh, kc, vc)
+        qb, ob = b.from_host(q), b.alloc_buffer(n * qh * 128 * 2)
+        gm = HipModel(b, synth.model_config(shape, 256, 64))
+        for layer, tid, fmt, data in synth.model_tensors(shape, 33):
+            gm.load_tensor(layer, tid, fmt, data)
+        prompt = [3, 99, 1500, 42]
+        gm.prefill(prompt, 0)
+        first = gm.read_argmax()
+        tokens = gm.decode_greedy(first, 4, 70)
+        size, slots, gen = b.scratch_info()
+        b.set_scratch_limit(size if kept else 64)
+        b.attention_prefill(ob, qb, kv, qh, base, n, 0)
+        _close(O.f32(b.download(ob, np.uint16, n * qh * 128)), want, "unsplit")
+        now = b.scratch_info()
+        assert now[0] == (size if kept else 0) and now[1] == slots and now[2] > gen
+        if not kept:
+            with pytest.raises(GhError) as e:
+                gm.decode_greedy(first, 4, 70)
+            assert e.value.code == -4  # GH_E_OOM
+        b.set_scratch_limit(0)
+        gm.prefill(prompt, 0)
+        assert np.array_equal(gm.decode_greedy(first, 4, 70), tokens)
+        b.attention_prefill(ob, qb, kv, qh, base, n, 0)
+        _close(O.f32(b.download(ob, np.uint16, n * qh * 128)), want, "split")
+        assert b.scratch_info()[0] > size
+        gm.close()
+        _free(b, qb, ob, kv.k, kv.v)
+
+
 def test_graph_replay_ignores_partials_of_earlier_steps(hip):
     """A replayed decode graph whose attention grid is fixed at 4 splits (forced: one step
     graph over the whole 256-position context), while the splits in use follow the position.
