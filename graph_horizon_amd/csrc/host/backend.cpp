@@ -1113,9 +1113,10 @@ static bool wide_tiles(const gh_backend* b, uint64_t tiles, uint64_t small, uint
     return 9 * 128 * ceil_div(tiles, (uint64_t)b->cus) <= 5 * br * ceil_div(small, (uint64_t)b->cus);
 }
 
-static GemmPlan plan_gemm(gh_backend* b, const gh_buf* w, uint32_t n) {
+// few = false: the tiles' plan, whose partials are smaller, also for few tokens.
+static GemmPlan plan_gemm(gh_backend* b, const gh_buf* w, uint32_t n, bool few = true) {
     const uint32_t rows = w->rows, units = w->cols / 64;
-    if (n <= kGemmFewMax) {
+    if (few && n <= kGemmFewMax) {
         const FewPlan f = plan_few(w->cols, n);
         return GemmPlan{(GhKernel)(f.k + (w->format == GH_FMT_Q4_K ? 0 : 1)), ceil_div(rows, 128), 1, f.splits, 0, f.shmem};
     }
@@ -1189,23 +1190,44 @@ static int gemm_kernel(gh_backend* b, const GemmPlan& p, uint64_t out, uint64_t 
     return launch(b, p.k, p.tr, p.tt, p.splits, gemm_block(p.k), &ga);
 }
 
+static int silu_launch(gh_backend* b, uint64_t out, uint64_t gate, uint64_t up, uint32_t n) {
+    GhEltArgs a{out, gate, up, n, (out | gate | up) % 16 == 0};
+    return launch(b, K_SILU_MUL, ceil_div(n, 2048), 1, 1, 256, &a);
+}
+
+static int gemv_f16(gh_backend* b, uint64_t out, const gh_buf* a, const gh_buf* w, uint32_t n) {
+    const GemvSeg seg{w, out, GH_EPI_F16};
+    return op_gemv(b, &seg, 1, a, n, 0, nullptr, 0, nullptr);
+}
+
 // One GEMM launch over its plan's tiles and K splits; with splits > 1 the kernel writes FP32
 // partials to the workspace and gh_gemm_reduce sums them in split order. `e` adds the SiLU
 // epilogue (in the GEMM or the reduce) or replaces the reduce by gh_gemm_tail (residual add
-// and RMSNorm of each output row).
+// and RMSNorm of each output row). Without memory for the few-token kernels' partials: below 8
+// tokens the GEMV (over exact weights too), which needs none, above the tiles, which need less.
 int op_gemm(gh_backend* b, uint64_t out, const gh_buf* a, const gh_buf* w, uint32_t n, const GemmEpi* e) {
     if (n < 8 && w->cols > 16384) return fail(b, GH_E_UNSUPPORTED, "gemv: in_dim above 16384");
-    const GemmPlan p = plan_gemm(b, w, n);
+    GemmPlan p = plan_gemm(b, w, n);
     const bool tail = e && e->resid;
     const uint32_t epi = e && !tail ? e->epi : GH_GEMM_EPI_F16;
     const uint64_t aux = e && !tail ? e->aux : 0;
+    bool gemv = false;
+    if (p.splits > 1 && p.shmem) {
+        bool room = false;
+        const int rc = try_workspace(b, (size_t)p.splits * n * w->rows * 4, &room);
+        if (rc) return rc;
+        gemv = !room && n < 8;
+        if (gemv) p.splits = 1;
+        else if (!room) p = plan_gemm(b, w, n, false);
+    }
     uint64_t part = 0;
     if (p.splits > 1) {
-        int rc = ensure_workspace(b, (size_t)p.splits * n * w->rows * 4);
+        const int rc = ensure_workspace(b, (size_t)p.splits * n * w->rows * 4);
         if (rc) return rc;
         part = (uint64_t)((char*)b->ws + kArgmaxBytes);
     }
-    int rc = gemm_kernel(b, p, out, part, a, w, n, epi, aux);
+    int rc = gemv ? gemv_f16(b, out, a, w, n) : gemm_kernel(b, p, out, part, a, w, n, epi, aux);
+    if (!rc && gemv && epi == GH_GEMM_EPI_SILU) rc = silu_launch(b, out, aux, out, n * w->rows);
     if (rc) return rc;
     GhGemmArgs ga{};
     ga.out = out;
@@ -1242,11 +1264,14 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
         return fail(b, GH_E_RANGE, "gemm swiglu: buffer too small");
     const FewPlan f = plan_few(wg->cols, std::min(n, kGemmFewMax));
     const uint64_t few_half = (uint64_t)f.splits * cells;
-    if (n <= kGemmFewMax && wg->rows % 4 == 0 && few_half <= 0xFFFFFFFFull) {
-        // few tokens: both matrices in one launch, partials [2][splits][n][rows] for the shared reduce
-        // (the second matrix's start is a 32-bit field)
-        int rc = ensure_workspace(b, 2 * few_half * 4);
+    // few tokens: both matrices in one launch, partials [2][splits][n][rows] for the shared reduce
+    // (the second matrix's start is a 32-bit field); without memory for them the launches below
+    bool few = n <= kGemmFewMax && wg->rows % 4 == 0 && few_half <= 0xFFFFFFFFull;
+    if (few) {
+        const int rc = try_workspace(b, 2 * few_half * 4, &few);
         if (rc) return rc;
+    }
+    if (few) {
         GhGemmArgs ga{};
         ga.x = a->addr;
         ga.part = (uint64_t)((char*)b->ws + kArgmaxBytes);
@@ -1258,11 +1283,18 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
         const uint32_t tiles = ceil_div(wg->rows, 128);
         ga.seg[0] = GhGemmSeg{wg->addr, 0, wg->rows, wg->format, 0, 0, 0, 0};
         ga.seg[1] = GhGemmSeg{wu->addr, 0, wg->rows, wu->format, tiles, 0, 0, (uint32_t)few_half};
-        rc = launch_few(b, f, ga, 2 * tiles);
+        const int rc = launch_few(b, f, ga, 2 * tiles);
         if (rc) return rc;
         ga.out = out->addr;
         return launch(b, K_GEMM_REDUCE_SWIGLU, (uint32_t)std::min<uint64_t>(ceil_div(cells / 4, (uint64_t)256), 4096),
                       1, 1, 256, &ga);
+    }
+    if (n < 8) {  // over exact weights still: one matrix at a time, down to the GEMV
+        GemmEpi e;
+        e.epi = GH_GEMM_EPI_SILU;
+        e.aux = gate->addr;
+        const int rc = op_gemm(b, gate->addr, a, wg, n);
+        return rc ? rc : op_gemm(b, out->addr, a, wu, n, &e);
     }
     // 49-128 tokens, Q4_K gate and up whose row pairs fill at most one wave of workgroups: one
     // launch of 96-row tiles (48 gate rows + the same 48 up rows) or, where those would be more
@@ -1289,7 +1321,7 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
     // picks them: 8B at 2048, 14B), so each sum is the separate launch's, over the FP16 copies
     // when both weights have one (8B 512-token prefill 11.73 -> 11.56-11.65 ms, same box; 96-row
     // pairs where the separate launches take 128 rows measured 34.6 -> 36.4 ms at 2048)
-    const GemmPlan pg = plan_gemm(b, wg, n), pu = plan_gemm(b, wu, n);
+    const GemmPlan pg = plan_gemm(b, wg, n, false), pu = plan_gemm(b, wu, n, false);
     const bool r96 = pg.k == K_GEMM4W_Q4K_R96 || pg.k == K_GEMM3_Q4K_R96;
     const bool r128 = pg.k == K_GEMM4W_Q4K_R128 || pg.k == K_GEMM3_Q4K_R128 || pg.k == K_GEMM5_Q4K;
     // Where the separate launches split K (8B at 129-255 tokens: 128 tiles x 2 splits and a
@@ -1405,8 +1437,22 @@ int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint3
     const bool tall = n >= kGemmTallTokens;
     bool copies = tall;
     for (uint32_t i = 0; i < nseg; ++i) copies = copies && b->w16.count(segs[i].w->addr);
-    const bool few = n <= kGemmFewMax;
-    const FewPlan fp = few ? plan_few(in_dim, n) : FewPlan{};
+    const FewPlan fp = plan_few(in_dim, std::min(n, kGemmFewMax));
+    bool few = n <= kGemmFewMax;
+    if (few && fp.splits > 1) {
+        const int rc = try_workspace(b, (size_t)fp.splits * n * total * 4, &few);
+        if (rc) return rc;
+        if (!few && n < 8) {  // without memory for the partials: the GEMV, over exact weights too
+            for (uint32_t i = 0; i < nseg; ++i) {
+                int rc = gemv_f16(b, segs[i].out->addr, a, segs[i].w, n);
+                if (!rc && segs[i].role)
+                    rc = op_rope(b, *rope, segs[i].out, segs[i].w->rows / head_dim, head_dim, base, n,
+                                 segs[i].role == GH_GEMM_ROLE_ROPE_QUERY ? GH_ROPE_QUERY : GH_ROPE_KEY, nullptr);
+                if (rc) return rc;
+            }
+            return GH_OK;
+        }
+    }
     const uint32_t tt = few ? 1 : ceil_div(n, tall ? 256u : 128u), units = in_dim / 64;
     // splits: the CUs over the tiles, at most 16 and at least 8 units per split (12 in the
     // 128-token tiles, as op_gemm), none empty
@@ -1500,12 +1546,7 @@ static int gemv_launch(gh_backend* b, const gh_buf* out, const gh_buf* a, const 
     // 4096 x 4096 Q4_K at 2 / 5 tokens 8.3 / 16.1 us against 9.6 / 10.2, 1024 x 4096 Q6_K 4.9 / 8.6
     // against 10.0 / 10.5, 12288 x 4096 14.9 / 32.7 against 13.3 / 13.4)
     const bool small = n < 8 && n * w->bytes <= (uint64_t)24 << 20;
-    if (!f32 && n >= kGemmMinTokens && !small) {
-        const int rc = op_gemm(b, out->addr, a, w, n);
-        if (rc != GH_E_OOM || n >= 8) return rc;
-        (void)hipGetLastError();  // no room for the partials: the GEMV needs none
-        b->err.clear();
-    }
+    if (!f32 && n >= kGemmMinTokens && !small) return op_gemm(b, out->addr, a, w, n);
     GemvSeg seg{w, out->addr, f32 ? (uint32_t)GH_EPI_F32 : (uint32_t)GH_EPI_F16};
     return op_gemv(b, &seg, 1, a, n, 0, nullptr, 0, nullptr);
 }
@@ -1577,8 +1618,7 @@ int gh_silu_mul(gh_backend* b, gh_encoder* enc, const gh_buf* out, const gh_buf*
     if (rc) return rc;
     if (!fits(out, (uint64_t)n * 2) || !fits(gate, (uint64_t)n * 2) || !fits(up, (uint64_t)n * 2))
         return latch(enc, fail(b, GH_E_RANGE, "silu_mul: buffer too small"));
-    GhEltArgs a{out->addr, gate->addr, up->addr, n, (out->addr | gate->addr | up->addr) % 16 == 0};
-    return latch(enc, launch(b, K_SILU_MUL, ceil_div(n, 2048), 1, 1, 256, &a));
+    return latch(enc, silu_launch(b, out->addr, gate->addr, up->addr, n));
 }
 
 int gh_residual_add(gh_backend* b, gh_encoder* enc, const gh_buf* x, const gh_buf* y,

@@ -247,3 +247,40 @@ def test_prefill_fp16_weight_copies_follow_reloaded_weights(hip):
     ref.close()
     assert not np.array_equal(before, want[0])  # the swap changes the result
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("n,limit", [(7, 0), (7, 4 << 20), (40, 6 << 20)])
+def test_short_prefill_without_scratch_for_its_partials(n, limit):
+    """A chunk of 2 to 48 rows whose split partials do not fit runs what needs less (the GEMV below 8
+    rows, the tiles' smaller split counts and the paired gate/up launch above) instead of failing: with
+    no workspace at all, with the 4 MB that a backend starts with (gate and up of 7 rows want 5.5), and
+    with 6 MB (Q/K/V of 40 rows want 7.9, gate and up 31, down 15.7)."""
+    from graph_horizon_amd import HipBackend
+    from graph_horizon_amd import _ffi as F
+
+    shape = dataclasses.replace(synth.SHAPES["8b"], name="8b-1", block_count=1, vocab_size=2048)
+    seed, base, rng = 29, 300, np.random.default_rng(29)
+    toks = [int(t) for t in rng.integers(0, shape.vocab_size, base + n)]
+    with HipBackend(0) as b:
+        gm = HipModel(b, synth.model_config(shape, base + n, prefill_rows=512))
+        for layer, tid, fmt, data in synth.model_tensors(shape, seed):
+            gm.load_tensor(layer, tid, fmt, data)
+        gm.prefill(toks[:base], 0)
+        # a growth (to 50 MB) that fails and leaves nothing
+        w = b.load_weight(F.FMT_Q4_K, synth.q4k_blocks(rng, 131072, 1024), 1024, 131072)
+        x, y = b.from_host(O.f16(rng.standard_normal(48 * 1024).astype(np.float32))), b.alloc_buffer(48 * 131072 * 2)
+        b.set_scratch_limit(64)
+        b.matmul_batched(y, x, w, 1024, 131072, 48)
+        assert b.scratch_info()[0] == 0
+        outs = []
+        for most in (limit or 64, 0):
+            b.set_scratch_limit(most)
+            gm.prefill(toks[base:], base)
+            kv, m = gm.kv(), (base + n) * shape.kv_head_count * shape.head_dim
+            outs.append([gm.read_logits(), gm.read_x()] +
+                        [b.download(c, np.uint16, m).view(np.float16).reshape(base + n, -1)[base:] for c in (kv.k, kv.v)])
+        gm.close()
+    for got, want, what in zip(outs[0], outs[1], ("logits", "x", "k", "v")):
+        got, want = got.astype(np.float64), want.astype(np.float64)
+        assert np.isfinite(got).all()
+        assert np.max(np.abs(got - want)) <= 2e-3 * max(np.abs(want).max(), 1.0), what
