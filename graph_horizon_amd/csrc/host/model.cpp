@@ -631,9 +631,10 @@ int gh_model_prefill(gh_model* m, const uint32_t* tokens, uint32_t n, uint32_t b
     if (urc) return urc;
     set_w16(m, copies);
     int rc = prefill_chunks(m, n, base);
-    if (rc == GH_E_OOM && copies && !m->w16.empty()) {
-        // the copies crowded out this prefill's workspace: drop them for good and run the
-        // prompt again dequantizing (every chunk rewrites the same cache rows)
+    if (rc == GH_E_OOM && !m->w16.empty()) {
+        // the copies (this prefill's or an earlier, longer one's) crowded out its workspace: drop
+        // them for good and run the prompt again dequantizing (every chunk rewrites the same cache
+        // rows)
         free_w16(m);
         m->w16_failed = true;
         m->b->err.clear();

@@ -284,3 +284,46 @@ def test_short_prefill_without_scratch_for_its_partials(n, limit):
         got, want = got.astype(np.float64), want.astype(np.float64)
         assert np.isfinite(got).all()
         assert np.max(np.abs(got - want)) <= 2e-3 * max(np.abs(want).max(), 1.0), what
+
+
+def test_short_prefill_gives_up_earlier_copies_for_its_workspace():
+    """A chunk of 100 rows reads no FP16 weight copies, but those that an earlier, longer prefill made
+    are what a device is full of: when the chunk's workspace cannot be had, they are freed and the chunk
+    is run again (which fails here, where the limit and not the memory is in the way)."""
+    import ctypes as C
+
+    from graph_horizon_amd import GhError, HipBackend
+    from graph_horizon_amd import _ffi as F
+
+    def free_memory():  # through the HIP runtime that the library is linked to
+        free, total = C.c_size_t(), C.c_size_t()
+        assert b.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    shape = dataclasses.replace(synth.SHAPES["8b"], name="8b-1", block_count=1, vocab_size=2048)
+    rng = np.random.default_rng(31)
+    toks = [int(t) for t in rng.integers(0, shape.vocab_size, 300)]
+    with HipBackend(0) as b:
+        gm = HipModel(b, synth.model_config(shape, 320, prefill_rows=512))
+        matrices = 0
+        for layer, tid, fmt, data in synth.model_tensors(shape, 31):
+            gm.load_tensor(layer, tid, fmt, data)
+            if layer != F.NO_LAYER and fmt in (F.FMT_Q4_K, F.FMT_Q6_K):
+                matrices += data.nbytes // (144 if fmt == F.FMT_Q4_K else 210) * 512  # bytes of its copy
+        gm.prefill(toks[:100], 0)
+        want = gm.read_logits()
+        gm.prefill(toks, 0)
+        # a growth (to 50 MB) that fails and leaves nothing
+        w = b.load_weight(F.FMT_Q4_K, synth.q4k_blocks(rng, 131072, 1024), 1024, 131072)
+        x, y = b.from_host(O.f16(rng.standard_normal(48 * 1024).astype(np.float32))), b.alloc_buffer(48 * 131072 * 2)
+        b.set_scratch_limit(64)
+        b.matmul_batched(y, x, w, 1024, 131072, 48)
+        free = free_memory()
+        with pytest.raises(GhError) as e:
+            gm.prefill(toks[:100], 0)
+        assert e.value.code == -4  # GH_E_OOM
+        assert free_memory() - free > 0.9 * matrices, matrices
+        b.set_scratch_limit(0)
+        gm.prefill(toks[:100], 0)
+        assert np.array_equal(gm.read_logits().view(np.uint32), want.view(np.uint32))
+        gm.close()
