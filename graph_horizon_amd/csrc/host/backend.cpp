@@ -1048,8 +1048,11 @@ namespace gh {
 // workgroups of 256 tokens, or 128 below 256 tokens, x 128 or 96 rows), over FP16 weight
 // copies where registered; K splits over the units when the tiles alone would leave CUs idle.
 constexpr uint32_t kGemmMinTokens = 2;
-// 12288 x 4096 at 48 / 64 tokens 25.7 / 33.4 us against 30.9 / 32.0 in the 128-token tiles, 4096 x 12288
-// 33.0 / 36.9 against 34.8 / 35.8
+// Single matrices: 12288 x 4096 at 48 / 64 tokens 25.7 / 33.4 us against 30.9 / 32.0 in the 128-token
+// tiles, 4096 x 12288 33.0 / 36.9 against 34.8 / 35.8. In the prefill driver at 48 rows, where gate and up
+// of the tiles are one unsplit launch: gate and up with their reduce 43.4 against 44.8 us (8B width), 63.4
+// against 63.7 (14B); Q/K/V 17.1 against 23.4 and 17.4 against 23.7; four blocks at 33 / 40 / 48 rows 521 /
+// 545 / 568 against 594 / 599 / 607 us (8B), 688 / 721 / 751 against 754 / 763 / 769 (14B).
 constexpr uint32_t kGemmFewMax = 48;
 constexpr uint32_t kGemmTailMaxRows = 8192;  // gh_gemm_tail: two 16-value items per thread
 
@@ -1063,8 +1066,10 @@ struct GemmPlan {
 };
 
 // The few-token kernels' launch: the Q4_K kernel for n tokens (+ 1: Q6_K, + 2: mixed), K splits and
-// dynamic LDS. Two blocks per split (both in flight from the start), more only past 32 splits, by
-// in_dim alone, so that a matrix's sums do not depend on the launch it is in.
+// dynamic LDS. Two blocks per split (both in flight from the start), more only past 32 splits, as many
+// as the LDS holds for n tokens; by in_dim and n alone, so that a matrix's sums do not depend on which of
+// these launches it is in. in_dim whose splits would still pass 32 (above 16384 at 48 tokens, 65536 at
+// 16) takes the tiles (at most 16): the partials grow with the splits, the work of a split does not.
 struct FewPlan {
     int k;
     uint32_t splits, shmem;
@@ -1079,6 +1084,10 @@ static FewPlan plan_few(uint32_t in_dim, uint32_t n) {
                   : n <= 16 ? K_GEMM_FEW_Q4K_T16
                   : n <= 32 ? K_GEMM_FEW_Q4K_T32 : K_GEMM_FEW_Q4K_T48;
     return FewPlan{k, splits, n * ((per * 256 + 8) + (per * 16 + 8)) * 2};
+}
+
+static bool few_applies(uint32_t in_dim, uint32_t n) {
+    return n >= kGemmMinTokens && n <= kGemmFewMax && plan_few(in_dim, n).splits <= 32;
 }
 
 // The few-token kernel over ga.seg[0 .. nseg), `tiles` row tiles of 128 in all.
@@ -1116,7 +1125,7 @@ static bool wide_tiles(const gh_backend* b, uint64_t tiles, uint64_t small, uint
 // few = false: the tiles' plan, whose partials are smaller, also for few tokens.
 static GemmPlan plan_gemm(gh_backend* b, const gh_buf* w, uint32_t n, bool few = true) {
     const uint32_t rows = w->rows, units = w->cols / 64;
-    if (few && n <= kGemmFewMax) {
+    if (few && few_applies(w->cols, n)) {
         const FewPlan f = plan_few(w->cols, n);
         return GemmPlan{(GhKernel)(f.k + (w->format == GH_FMT_Q4_K ? 0 : 1)), ceil_div(rows, 128), 1, f.splits, 0, f.shmem};
     }
@@ -1266,7 +1275,7 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
     const uint64_t few_half = (uint64_t)f.splits * cells;
     // few tokens: both matrices in one launch, partials [2][splits][n][rows] for the shared reduce
     // (the second matrix's start is a 32-bit field); without memory for them the launches below
-    bool few = n <= kGemmFewMax && wg->rows % 4 == 0 && few_half <= 0xFFFFFFFFull;
+    bool few = few_applies(wg->cols, n) && wg->rows % 4 == 0 && few_half <= 0xFFFFFFFFull;
     if (few) {
         const int rc = try_workspace(b, 2 * few_half * 4, &few);
         if (rc) return rc;
@@ -1438,7 +1447,7 @@ int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint3
     bool copies = tall;
     for (uint32_t i = 0; i < nseg; ++i) copies = copies && b->w16.count(segs[i].w->addr);
     const FewPlan fp = plan_few(in_dim, std::min(n, kGemmFewMax));
-    bool few = n <= kGemmFewMax;
+    bool few = few_applies(in_dim, n);
     if (few && fp.splits > 1) {
         const int rc = try_workspace(b, (size_t)fp.splits * n * total * 4, &few);
         if (rc) return rc;

@@ -141,6 +141,21 @@ def test_gemm_few_tokens(hip, fmt, rows, in_dim, n):
     _check_fp64(fmt, w, a16, got, rows, in_dim, n, f"{fmt} {rows}x{in_dim} n={n}", f16_weights=n >= 8)
 
 
+@pytest.mark.parametrize("in_dim,n,most", [
+    (65536, 16, 32),  # the most blocks per split (eight, 70 KB of LDS)
+    (65536, 48, 16), (16640, 48, 16),  # two blocks per split would be 128 and 33 splits: the tiles instead
+])
+def test_gemm_few_tokens_bounds_its_splits(in_dim, n, most):
+    """The partials of deep matrices stay within 32 splits (16 in the tiles), and the sums right."""
+    from graph_horizon_amd import HipBackend
+
+    fmt, rows = F.FMT_Q4_K, 768 if in_dim == 65536 else 3000
+    with HipBackend(0) as b:
+        w, a16, got = _run(b, fmt, rows, in_dim, n, in_dim + n)
+        assert b.scratch_info()[0] <= max(4 << 20, most * n * rows * 4 + 4096)
+    _check_fp64(fmt, w, a16, got, rows, in_dim, n, f"{rows}x{in_dim} n={n}")
+
+
 @pytest.mark.parametrize("fmt", [F.FMT_Q4_K, F.FMT_Q6_K], ids=["q4k", "q6k"])
 @pytest.mark.parametrize("x_scale", [2.0 ** -20, 2.0 ** -10, 400.0])
 def test_gemm_few_tokens_exact_extremes(hip, fmt, x_scale):
