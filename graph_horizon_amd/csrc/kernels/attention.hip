@@ -623,7 +623,7 @@ __device__ __forceinline__ uint32_t kv_at(uint32_t r, uint32_t blk) { return r *
 // lane i of a load lands at byte 16 i of its 1 KiB destination, four 256-byte rows): wave w
 // loads rows 16 w .. 16 w + 15, lane i of load q the 16-byte chunk of row r = 16 w + 4 q + i / 16
 // that belongs in slot i mod 16. Keys past kv_end (masked; their weight is 0) re-read key
-// kv_end - 1, so every value in the tile is a finite cache value and no load leaves the range.
+// kv_end - 1, so the tile holds only rows that the block attends and no load leaves the range.
 // The loads are issued from inline assembly: the compiler does not count them, so it adds no
 // wait before the reads of the other tile buffer; the caller waits (vmcnt(0)) before the
 // barrier that hands the tile over. (Untracked loads can only make the compiler's own waits
@@ -692,6 +692,58 @@ typedef _Float16 ah2 __attribute__((ext_vector_type(2)));
 // ceil(tiles of the last block / splits) of them
 __device__ __forceinline__ uint32_t attn_tiles(const GhAttnArgs& a, uint32_t qb, uint32_t pq) {
     return (a.base + min((qb + 1) * pq, a.rows) + kPK - 1) / kPK;
+}
+
+// Query row r of head h over keys k0 .. k1 - 1 (those that it sees) by one wave: lanes are keys for the
+// scores, pairs of value dims for the sum. FP32 weights, and no V row but the keys' own. For
+// rows that the tiles cannot give (attn_prefill); its speed does not matter.
+template <bool SPLIT>
+__device__ __forceinline__ void attn_row(const GhAttnArgs& a, const uint16_t* kc, const uint16_t* vc, uint32_t kv_row,
+                                         uint32_t r, uint32_t h, uint32_t k0, uint32_t k1, float sl2) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t head = (uint64_t)r * a.q_heads + h;
+    const GH_GLOBAL uint4* qp = gh_gp<uint4>(a.q + head * 256);
+    float m = -__builtin_inff(), l = 0.0f, o0 = 0.0f, o1 = 0.0f;
+    for (uint32_t c = k0; c < k1; c += 64) {
+        const GH_GLOBAL uint4* kp = gh_gp<uint4>((uint64_t)(uintptr_t)(kc + (size_t)min(c + lane, k1 - 1) * kv_row));
+        float s = 0.0f;
+#pragma unroll 2
+        for (uint32_t i = 0; i < 16; ++i) {
+            const uint4 q = qp[i], k = kp[i];
+            s = gh_dot2(q.x, k.x, s);
+            s = gh_dot2(q.y, k.y, s);
+            s = gh_dot2(q.z, k.z, s);
+            s = gh_dot2(q.w, k.w, s);
+        }
+        s = c + lane < k1 ? s : -__builtin_inff();
+        const float m_new = fmaxf(m, gh_wave_max(s) * sl2);
+        const float ref = m_new == -__builtin_inff() ? 0.0f : m_new;
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s, sl2, -ref)), f = __builtin_amdgcn_exp2f(m - ref);
+        m = m_new;
+        l = l * f + p;
+        o0 *= f;
+        o1 *= f;
+        const uint32_t n = min(64u, k1 - c);
+        for (uint32_t i = 0; i < n; ++i) {
+            const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), i));
+            const uint32_t v = gh_gp<uint32_t>((uint64_t)(uintptr_t)(vc + (size_t)(c + i) * kv_row))[lane];
+            o0 += w * gh_h2f(v & 0xFFFFu);
+            o1 += w * gh_h2f(v >> 16);
+        }
+    }
+    l = gh_wave_sum(l);
+    if constexpr (SPLIT) {
+        const uint64_t pi = head * a.splits + blockIdx.z;
+        if (lane == 0) {
+            gh_gpw<float>(a.part_m)[pi] = m;
+            gh_gpw<float>(a.part_l)[pi] = l;
+        }
+        gh_gpw<float>(a.part_acc)[pi * 128 + 2 * lane] = o0;
+        gh_gpw<float>(a.part_acc)[pi * 128 + 2 * lane + 1] = o1;
+    } else {
+        const float inv = 1.0f / l;
+        gh_gpw<uint32_t>(a.out)[head * 64 + lane] = (uint32_t)gh_f2h(o0 * inv) | ((uint32_t)gh_f2h(o1 * inv) << 16);
+    }
 }
 
 // QT: query tiles of 16 rows per wave; G: query heads per kv head; SPLIT: key splits (the plain
@@ -856,12 +908,27 @@ __device__ __forceinline__ void attn_prefill(const GhAttnArgs& a) {
     uint32_t tile = tile0;
     for (; tile < ntiles && tile * kPK + kPK - 1 <= first_pos; ++tile) step(tile, Flag<false>{});
     for (; tile < ntiles; ++tile) step(tile, Flag<true>{});
+    // The products take in every V row of a tile: a key past a query's own has weight 0, but 0 times an
+    // infinity or a NaN is not 0, and the two parts of a weight do not add up against an infinity. What
+    // such a V leaves in a row stays non-finite, so these rows are found here and computed again below.
+    uint32_t again[QT];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        float z = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z = __builtin_fmaf(o[j][t][e], 0.0f, z);
+        uint64_t lanes = __ballot(z != 0.0f);  // a NaN
+        lanes |= lanes >> 32;
+        again[t] = (uint32_t)(lanes | lanes >> 16) & 0xFFFFu;
+    }
     // O^T tile (j, t): lane holds dims 16 j + 4 fg + e of query row qw + 16 t + fr
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
         const uint32_t r = qw + 16 * t + fr;
         const float lt = xor_sum(l[t]);
-        if (r >= a.rows) continue;
+        if (r >= a.rows || (again[t] >> fr & 1u)) continue;
         if constexpr (SPLIT) {
             const uint64_t pi = ((uint64_t)r * a.q_heads + h) * a.splits + blockIdx.z;
             if (fg == 0) {
@@ -882,6 +949,13 @@ __device__ __forceinline__ void attn_prefill(const GhAttnArgs& a) {
             *(GH_GLOBAL uint2*)(op + 16 * j) = make_uint2(w0, w1);
         }
     }
+#pragma unroll
+    for (int t = 0; t < QT; ++t)
+        for (uint32_t rows = again[t]; rows; rows &= rows - 1) {  // wave-uniform
+            const uint32_t r = qw + 16 * t + __builtin_ctz(rows);
+            if (r < a.rows)
+                attn_row<SPLIT>(a, kc, vc, kv_row32, r, h, tile0 * kPK, min(ntiles * kPK, a.base + r + 1), sl2);
+        }
 }
 }  // namespace
 
@@ -923,7 +997,8 @@ GH_KERNEL __launch_bounds__(256) void gh_attn_merge(GhAttnArgs a) {
         for (uint32_t i = 0; i < 8; ++i) p[i] = pa[(uint64_t)min(s0 + i, ns - 1) * 64];
 #pragma unroll
         for (uint32_t i = 0; i < 8; ++i) {
-            const float ws = s0 + i < ns ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s0 + i)) : 0.0f;
+            if (s0 + i >= ns) break;  // wave-uniform; the last split again, whose sum may be infinite
+            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s0 + i));
             o.x += ws * p[i].x;
             o.y += ws * p[i].y;
         }

@@ -111,6 +111,42 @@ def test_prefill_attention_groups_rows_and_key_splits(hip, qh, kvh, base, n):
     _free(hip, qb, ob, kv.k, kv.v)
 
 
+@pytest.mark.parametrize("qh,kvh", [(8, 8), (16, 8), (32, 8), (64, 8)], ids=["g1", "g2", "g4", "g8"])
+@pytest.mark.parametrize("base,n", [(1000, 5), (100, 40), (40, 600)])
+def test_prefill_attention_non_finite_cache_rows(hip, qh, kvh, base, n):
+    """An infinity or a NaN in the cache reaches the rows that see its position and no others: not the
+    earlier rows of the same chunk, whose key tile holds it too, and not from slots past the chunk. 16-
+    and 32-row query blocks, with and without key splits."""
+    if n == 600 and qh == 8:
+        n = 2050
+    rng = np.random.default_rng(qh + base + n)
+    ctx, at, last = base + n + 3, base + n // 2, base + n - 1
+    kc = rng.standard_normal((ctx, kvh, 128)).astype(np.float32)
+    vc = rng.standard_normal((ctx, kvh, 128)).astype(np.float32)
+    vc[at, :, 0], vc[at, :, 1], vc[at, 0, 2] = np.inf, np.nan, -np.inf
+    kc[last, 1, 5] = np.nan
+    kc[base + n:], vc[base + n:] = np.nan, np.nan
+    kc, vc = O.f16(kc.reshape(-1)), O.f16(vc.reshape(-1))
+    q = O.f16(rng.standard_normal(n * qh * 128).astype(np.float32))
+    kv = _kv(hip, 1, ctx, kvh, kc, vc)
+    qb, ob = hip.from_host(q), hip.alloc_buffer(n * qh * 128 * 2)
+    want = O.f32(O.attention_prefill(q, kc, vc, 128, kvh, qh, base, n, 0, ctx))
+    finite = np.isfinite(want)
+    seen = finite.reshape(n, -1).all(axis=1)
+    assert seen[:at - base].all() and not seen[at - base:].any()
+    try:
+        for splits in (0, 1, 3):
+            hip.set_attention_splits(splits)
+            hip.attention_prefill(ob, qb, kv, qh, base, n, 0)
+            got = O.f32(hip.download(ob, np.uint16, n * qh * 128))
+            assert np.array_equal(np.isnan(got), np.isnan(want)), splits
+            assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]), splits
+            _close(got[finite], want[finite], f"splits {splits}")
+    finally:
+        hip.set_attention_splits(0)
+    _free(hip, qb, ob, kv.k, kv.v)
+
+
 def _reference_case(ctx_total):
     """attention_prefill_decode_for_scheme inputs (vulkan/mod.rs:955-1000), one layer."""
     qh, hd = 4, 128
