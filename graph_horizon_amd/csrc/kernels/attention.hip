@@ -596,6 +596,11 @@ GH_KERNEL __launch_bounds__(64) void gh_xcd_probe(uint64_t out, uint32_t gx, uin
 //                   which leaves the product unchanged). P is split into FP16 hi + lo parts
 //                   (two MFMAs), so P·V carries FP32-level accuracy.
 // Softmax in base 2: scores are scaled by scale·log2(e), p = 2^(s - m), rescale 2^(m_old - m).
+// m is the running maximum less kUp: the parts of a weight end at 2^-25, so with G = 1 and 2, whose
+// decode kernel holds its weights in FP32, the largest is 2^15 and not 1, and the parts reach 2^-40 of
+// it. (As with 1, a weight below 2^-25 of the largest would count in the denominator alone: a key
+// against 32768 of 2^-26 each lost a numerator of 2^-11. With 4 and 8, the decode kernel's parts
+// are the same as here.)
 // Rows: query r at position base + r attends positions 0..base + r (the reference's prefill,
 // attention/mod.rs:582-725). Query blocks run heaviest (latest) first.
 // Key splits (a.splits > 1): where the query blocks alone leave CUs idle (few rows), split z of
@@ -694,10 +699,13 @@ __device__ __forceinline__ uint32_t attn_tiles(const GhAttnArgs& a, uint32_t qb,
     return (a.base + min((qb + 1) * pq, a.rows) + kPK - 1) / kPK;
 }
 
+template <int G>
+constexpr float kUp = G < 4 ? 15.0f : 0.0f;
+
 // Query row r of head h over keys k0 .. k1 - 1 (those that it sees) by one wave: lanes are keys for the
 // scores, pairs of value dims for the sum. FP32 weights, and no V row but the keys' own. For
 // rows that the tiles cannot give (attn_prefill); its speed does not matter.
-template <bool SPLIT>
+template <int G, bool SPLIT>
 __device__ __forceinline__ void attn_row(const GhAttnArgs& a, const uint16_t* kc, const uint16_t* vc, uint32_t kv_row,
                                          uint32_t r, uint32_t h, uint32_t k0, uint32_t k1, float sl2) {
     const uint32_t lane = threadIdx.x & 63u;
@@ -716,7 +724,7 @@ __device__ __forceinline__ void attn_row(const GhAttnArgs& a, const uint16_t* kc
             s = gh_dot2(q.w, k.w, s);
         }
         s = c + lane < k1 ? s : -__builtin_inff();
-        const float m_new = fmaxf(m, gh_wave_max(s) * sl2);
+        const float m_new = fmaxf(m, __builtin_fmaf(gh_wave_max(s), sl2, -kUp<G>));
         const float ref = m_new == -__builtin_inff() ? 0.0f : m_new;
         const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s, sl2, -ref)), f = __builtin_amdgcn_exp2f(m - ref);
         m = m_new;
@@ -860,7 +868,7 @@ __device__ __forceinline__ void attn_prefill(const GhAttnArgs& a) {
             // its split (only in masked tiles: a later split's first tile may lie past the row)
             // m is -inf, and the exponents are taken from 0 so that every weight and the
             // rescale come out as 0, not NaN.
-            float m_new = fmaxf(m[t], xor_max(mx) * sl2);
+            float m_new = fmaxf(m[t], G < 4 ? __builtin_fmaf(xor_max(mx), sl2, -kUp<G>) : xor_max(mx) * sl2);
             const float m_old = m[t];
             m[t] = m_new;
             if constexpr (SPLIT && kMask) m_new = m_new == -__builtin_inff() ? 0.0f : m_new;
@@ -954,7 +962,7 @@ __device__ __forceinline__ void attn_prefill(const GhAttnArgs& a) {
         for (uint32_t rows = again[t]; rows; rows &= rows - 1) {  // wave-uniform
             const uint32_t r = qw + 16 * t + __builtin_ctz(rows);
             if (r < a.rows)
-                attn_row<SPLIT>(a, kc, vc, kv_row32, r, h, tile0 * kPK, min(ntiles * kPK, a.base + r + 1), sl2);
+                attn_row<G, SPLIT>(a, kc, vc, kv_row32, r, h, tile0 * kPK, min(ntiles * kPK, a.base + r + 1), sl2);
         }
 }
 }  // namespace

@@ -147,6 +147,44 @@ def test_prefill_attention_non_finite_cache_rows(hip, qh, kvh, base, n):
     _free(hip, qb, ob, kv.k, kv.v)
 
 
+@pytest.mark.parametrize("qh,kvh", [(8, 8), (16, 8)], ids=["g1", "g2"])
+@pytest.mark.parametrize("gap", [26, 34])
+def test_prefill_attention_long_flat_tail(hip, qh, kvh, gap):
+    """One key far above 32768 others, whose weights are 2^-gap of its: together 2^-11 of the sum (or
+    2^-19), all of the numerator where the large key's V is 0. Against fp64, with and without key splits
+    and as the decode kernel gives each row. Bar: the output's FP16 rounding (2^-11 relative; 2^-25 where it
+    is subnormal), and 2^-40 of the largest weight lost per key, both parts' ends: 2^(gap - 40) of each."""
+    n, base = 24, 32768
+    ctx = base + n
+    # q is ones, so a key's score is the sum of its values / sqrt(128)
+    step = gap * np.log(2.0) * np.sqrt(128.0) / 128
+    kc = np.full((ctx, kvh, 128), -step, np.float32)
+    kc[7] = 0.0
+    vc = np.full((ctx, kvh, 128), 48.0, np.float32)
+    vc[7] = 0.0
+    q = np.ones(n * qh * 128, np.float32)
+    k16, v16, q16 = O.f16(kc.reshape(-1)), O.f16(vc.reshape(-1)), O.f16(q)
+    kv = _kv(hip, 1, ctx, kvh, k16, v16)
+    qb, ob = hip.from_host(q16), hip.alloc_buffer(n * qh * 128 * 2)
+    s = O.f32(k16[:128]).astype(np.float64).sum() / np.sqrt(128.0)  # the others' score
+    tail = np.exp(s) * (base + np.arange(n))  # of base + r keys beside key 7
+    want = np.repeat(48.0 * tail / (1.0 + tail), qh * 128)
+    tol = want * (2.0 ** -11 + 2.0 ** (gap - 40) + 1e-5) + 2.0 ** -25
+    try:
+        for splits in (0, 1):
+            hip.set_attention_splits(splits)
+            hip.attention_prefill(ob, qb, kv, qh, base, n, 0)
+            got = O.f32(hip.download(ob, np.uint16, n * qh * 128)).astype(np.float64)
+            worst = np.max(np.abs(got - want) / tol)
+            assert worst <= 1, (splits, worst)
+    finally:
+        hip.set_attention_splits(0)
+    hip.attention_decode(ob, qb, kv, qh, base, 0)
+    got = O.f32(hip.download(ob, np.uint16, qh * 128)).astype(np.float64)
+    assert np.max(np.abs(got - want[:qh * 128]) / tol[:qh * 128]) <= 1
+    _free(hip, qb, ob, kv.k, kv.v)
+
+
 def _reference_case(ctx_total):
     """attention_prefill_decode_for_scheme inputs (vulkan/mod.rs:955-1000), one layer."""
     qh, hd = 4, 128
