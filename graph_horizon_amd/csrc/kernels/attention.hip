@@ -702,18 +702,22 @@ __device__ __forceinline__ uint32_t attn_tiles(const GhAttnArgs& a, uint32_t qb,
 template <int G>
 constexpr float kUp = G < 4 ? 15.0f : 0.0f;
 
-// Query row r of head h over keys k0 .. k1 - 1 (those that it sees) by one wave: lanes are keys for the
-// scores, pairs of value dims for the sum. FP32 weights, and no V row but the keys' own. For
-// rows that the tiles cannot give (attn_prefill); its speed does not matter.
-template <int G, bool SPLIT>
-__device__ __forceinline__ void attn_row(const GhAttnArgs& a, const uint16_t* kc, const uint16_t* vc, uint32_t kv_row,
-                                         uint32_t r, uint32_t h, uint32_t k0, uint32_t k1, float sl2) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t head = (uint64_t)r * a.q_heads + h;
+// Query row r of head h by one wave and over its own keys alone: lanes are keys for the scores, pairs of
+// value dims for the sum, with FP32 weights. For the rows that the tiles cannot give: their products take in
+// every V row of a tile, and a key past a query's own has weight 0, but 0 times an infinity or a NaN is not 0
+// (nor do the two parts of a weight add up against an infinity). What such a V leaves in a row's sums
+// stays non-finite, so the kernels that write outputs look for that and come here; a row that sees the
+// value itself gets it again. Speed does not matter here.
+__device__ __forceinline__ void attn_row(const GhAttnArgs& a, uint32_t r, uint32_t h) {
+    const uint32_t lane = threadIdx.x & 63u, k1 = a.base + r + 1;
+    const uint64_t head = (uint64_t)r * a.q_heads + h, kv_row = (uint64_t)a.kv_heads * 256;  // bytes
+    const uint64_t cache0 = (uint64_t)a.layer * a.context * kv_row + h / (a.q_heads / a.kv_heads) * 256;
+    const uint64_t kc = a.kc + cache0, vc = a.vc + cache0;
+    const float sl2 = a.scale * 1.4426950408889634f;
     const GH_GLOBAL uint4* qp = gh_gp<uint4>(a.q + head * 256);
     float m = -__builtin_inff(), l = 0.0f, o0 = 0.0f, o1 = 0.0f;
-    for (uint32_t c = k0; c < k1; c += 64) {
-        const GH_GLOBAL uint4* kp = gh_gp<uint4>((uint64_t)(uintptr_t)(kc + (size_t)min(c + lane, k1 - 1) * kv_row));
+    for (uint32_t c = 0; c < k1; c += 64) {
+        const GH_GLOBAL uint4* kp = gh_gp<uint4>(kc + min(c + lane, k1 - 1) * kv_row);
         float s = 0.0f;
 #pragma unroll 2
         for (uint32_t i = 0; i < 16; ++i) {
@@ -723,10 +727,10 @@ __device__ __forceinline__ void attn_row(const GhAttnArgs& a, const uint16_t* kc
             s = gh_dot2(q.z, k.z, s);
             s = gh_dot2(q.w, k.w, s);
         }
-        s = c + lane < k1 ? s : -__builtin_inff();
-        const float m_new = fmaxf(m, __builtin_fmaf(gh_wave_max(s), sl2, -kUp<G>));
+        s = c + lane < k1 ? s * sl2 : -__builtin_inff();
+        const float m_new = fmaxf(m, gh_wave_max(s));
         const float ref = m_new == -__builtin_inff() ? 0.0f : m_new;
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s, sl2, -ref)), f = __builtin_amdgcn_exp2f(m - ref);
+        const float p = __builtin_amdgcn_exp2f(s - ref), f = __builtin_amdgcn_exp2f(m - ref);
         m = m_new;
         l = l * f + p;
         o0 *= f;
@@ -734,24 +738,13 @@ __device__ __forceinline__ void attn_row(const GhAttnArgs& a, const uint16_t* kc
         const uint32_t n = min(64u, k1 - c);
         for (uint32_t i = 0; i < n; ++i) {
             const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), i));
-            const uint32_t v = gh_gp<uint32_t>((uint64_t)(uintptr_t)(vc + (size_t)(c + i) * kv_row))[lane];
+            const uint32_t v = gh_gp<uint32_t>(vc + (c + i) * kv_row)[lane];
             o0 += w * gh_h2f(v & 0xFFFFu);
             o1 += w * gh_h2f(v >> 16);
         }
     }
-    l = gh_wave_sum(l);
-    if constexpr (SPLIT) {
-        const uint64_t pi = head * a.splits + blockIdx.z;
-        if (lane == 0) {
-            gh_gpw<float>(a.part_m)[pi] = m;
-            gh_gpw<float>(a.part_l)[pi] = l;
-        }
-        gh_gpw<float>(a.part_acc)[pi * 128 + 2 * lane] = o0;
-        gh_gpw<float>(a.part_acc)[pi * 128 + 2 * lane + 1] = o1;
-    } else {
-        const float inv = 1.0f / l;
-        gh_gpw<uint32_t>(a.out)[head * 64 + lane] = (uint32_t)gh_f2h(o0 * inv) | ((uint32_t)gh_f2h(o1 * inv) << 16);
-    }
+    const float inv = 1.0f / gh_wave_sum(l);
+    gh_gpw<uint32_t>(a.out)[head * 64 + lane] = (uint32_t)gh_f2h(o0 * inv) | ((uint32_t)gh_f2h(o1 * inv) << 16);
 }
 
 // QT: query tiles of 16 rows per wave; G: query heads per kv head; SPLIT: key splits (the plain
@@ -916,20 +909,20 @@ __device__ __forceinline__ void attn_prefill(const GhAttnArgs& a) {
     uint32_t tile = tile0;
     for (; tile < ntiles && tile * kPK + kPK - 1 <= first_pos; ++tile) step(tile, Flag<false>{});
     for (; tile < ntiles; ++tile) step(tile, Flag<true>{});
-    // The products take in every V row of a tile: a key past a query's own has weight 0, but 0 times an
-    // infinity or a NaN is not 0, and the two parts of a weight do not add up against an infinity. What
-    // such a V leaves in a row stays non-finite, so these rows are found here and computed again below.
-    uint32_t again[QT];
+    // rows with a non-finite sum (attn_row); with key splits gh_attn_merge sees to them
+    uint32_t again[QT] = {};
+    if constexpr (!SPLIT) {
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-        float z = 0.0f;
+        for (int t = 0; t < QT; ++t) {
+            af4 z = o[0][t] * 0.0f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
+            for (int j = 1; j < 8; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) z = __builtin_fmaf(o[j][t][e], 0.0f, z);
-        uint64_t lanes = __ballot(z != 0.0f);  // a NaN
-        lanes |= lanes >> 32;
-        again[t] = (uint32_t)(lanes | lanes >> 16) & 0xFFFFu;
+                for (int e = 0; e < 4; ++e) z[e] = __builtin_fmaf(o[j][t][e], 0.0f, z[e]);
+            uint64_t lanes = __ballot(z[0] + z[1] + z[2] + z[3] != 0.0f);  // a NaN
+            lanes |= lanes >> 32;
+            again[t] = (uint32_t)(lanes | lanes >> 16) & 0xFFFFu;
+        }
     }
     // O^T tile (j, t): lane holds dims 16 j + 4 fg + e of query row qw + 16 t + fr
 #pragma unroll
@@ -957,13 +950,14 @@ __device__ __forceinline__ void attn_prefill(const GhAttnArgs& a) {
             *(GH_GLOBAL uint2*)(op + 16 * j) = make_uint2(w0, w1);
         }
     }
-#pragma unroll
-    for (int t = 0; t < QT; ++t)
-        for (uint32_t rows = again[t]; rows; rows &= rows - 1) {  // wave-uniform
-            const uint32_t r = qw + 16 * t + __builtin_ctz(rows);
-            if (r < a.rows)
-                attn_row<G, SPLIT>(a, kc, vc, kv_row32, r, h, tile0 * kPK, min(ntiles * kPK, a.base + r + 1), sl2);
+    if constexpr (!SPLIT) {
+        uint32_t rows = again[0];
+        if constexpr (QT == 2) rows |= again[1] << 16;
+        for (; __builtin_expect(rows != 0, 0); rows &= rows - 1) {  // wave-uniform
+            const uint32_t r = qw + __builtin_ctz(rows);
+            if (r < a.rows) attn_row(a, r, h);
         }
+    }
 }
 }  // namespace
 
@@ -1005,11 +999,14 @@ GH_KERNEL __launch_bounds__(256) void gh_attn_merge(GhAttnArgs a) {
         for (uint32_t i = 0; i < 8; ++i) p[i] = pa[(uint64_t)min(s0 + i, ns - 1) * 64];
 #pragma unroll
         for (uint32_t i = 0; i < 8; ++i) {
-            if (s0 + i >= ns) break;  // wave-uniform; the last split again, whose sum may be infinite
-            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s0 + i));
+            const float ws = s0 + i < ns ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s0 + i)) : 0.0f;
             o.x += ws * p[i].x;
             o.y += ws * p[i].y;
         }
+    }
+    if (__builtin_expect(__ballot(o.x * 0.0f + o.y * 0.0f != 0.0f) != 0, 0)) {  // a NaN: not finite
+        attn_row(a, pair / a.q_heads, pair % a.q_heads);
+        return;
     }
     gh_gpw<uint32_t>(a.out)[(uint64_t)pair * 64 + lane] =
         (uint32_t)gh_f2h(o.x) | ((uint32_t)gh_f2h(o.y) << 16);
