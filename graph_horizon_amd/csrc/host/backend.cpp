@@ -1083,7 +1083,8 @@ static FewPlan plan_few(uint32_t in_dim, uint32_t n) {
     const int k = n < 8     ? K_GEMM_FEW_Q4K_T8
                   : n <= 16 ? K_GEMM_FEW_Q4K_T16
                   : n <= 32 ? K_GEMM_FEW_Q4K_T32 : K_GEMM_FEW_Q4K_T48;
-    return FewPlan{k, splits, n * ((per * 256 + 8) + (per * 16 + 8)) * 2};
+    // the activations' rows and, below 8 tokens, the sub-block means' (gemm_few.hip)
+    return FewPlan{k, splits, n * ((per * 256 + 8) + (n < 8 ? per * 32 + 8 : 0)) * 2};
 }
 
 static bool few_applies(uint32_t in_dim, uint32_t n) {

@@ -17,8 +17,9 @@
 // matrix cores sum a whole block of x · (scale · quant), and the FP16 block scale enters once per
 // block in FP32:
 //   Q4_K: scale · quant <= 63 · 15 = 945; the minima as one more product over the block's eight
-//     sub-blocks, min_j · Σx_j: Σx_j goes in as hi + 2^-11 mid FP16 parts of the sub-block's mean
-//     (22 bits or more of its FP32 value), so Σ = d · S - 32 dmin · M;
+//     sub-blocks, min_j · Σx_j: Σx_j, an FP32 sum, goes in as the FP16 parts hi + 2^-11 mid + 2^-22 low
+//     of the sub-block's mean, which hold all of it (33 bits; where a part is subnormal, down to 2^-46,
+//     and a mean of 32 FP16 values is a multiple of 2^-29), so Σ = d · S - 32 dmin · M;
 //   Q6_K: |scale · (quant - 32)| <= 4096, of which FP16 holds all up to 2048 and the even ones; the
 //     +-1 that rounding leaves out goes in as a second product.
 // There quants are used as FP16 subnormals (the integer q in the low bits is q · 2^-24), multiplied
@@ -96,8 +97,8 @@ __device__ __forceinline__ uint2 q6_scales(const uint4& sc, uint32_t u) {
 
 // The staged activations: row t (token) holds the split's k in 8-value chunks, for EXACT with the
 // values in the order 0 2 1 3 4 6 5 7 that its quant dwords unpack to; `xp` halves a row. Sub-block
-// means (EXACT Q4_K): for token t, block b and unit u the hi and mid parts of its two sub-blocks,
-// 4 halves at sums + t · sp + 16 b + 4 u.
+// means (EXACT Q4_K): for token t, block b and unit u the hi, mid and low parts (and a zero) of its two
+// sub-blocks, 8 halves at sums + t · sp + 32 b + 8 u.
 struct Staged {
     const _Float16* xs;
     const _Float16* sums;
@@ -197,8 +198,7 @@ __device__ __forceinline__ void block_exact(const Unit<FMT> (&w)[2], const Stage
     f4v S[2][1] = {{f4v{}}, {f4v{}}};
     uint32_t p[2][8], q[2][8];
     if constexpr (FMT == kQ4K) {
-        uint32_t s0[2], s1[2];
-        h8 mv[2];
+        uint32_t s0[2], s1[2], mn[2];  // mn: the two minima
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             uint32_t sc0, mn0, sc1, mn1;
@@ -207,9 +207,8 @@ __device__ __forceinline__ void block_exact(const Unit<FMT> (&w)[2], const Stage
             const _Float16 a = (_Float16)(float)(sc0 << 10), b = (_Float16)(float)(sc1 << 6);
             s0[r] = __builtin_bit_cast(uint32_t, gh_h2{a, a});
             s1[r] = __builtin_bit_cast(uint32_t, gh_h2{b, b});
-            const _Float16 z = (_Float16)0.0f, m0 = (_Float16)(float)mn0, m1 = (_Float16)(float)mn1;
-            const _Float16 e = (_Float16)0.00048828125f;  // 2^-11
-            mv[r] = h8{m0, m0 * e, m1, m1 * e, z, z, z, z};
+            mn[r] = __builtin_bit_cast(uint32_t, gh_h2{(_Float16)(float)mn0, (_Float16)(float)mn1});
+            asm volatile("" : "+v"(mn[r]));  // one register until the sums' product below
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -229,11 +228,14 @@ __device__ __forceinline__ void block_exact(const Unit<FMT> (&w)[2], const Stage
             mma16<1>(xr, 32 + 16 * h, q[0], q[1], S);
             __builtin_amdgcn_sched_barrier(0);  // one half's fragments live at a time
         }
-        const uint2 sm = *(const uint2*)(st.sums + row * st.sp + 16 * at + 4 * u);
-        const h8 x = __builtin_bit_cast(h8, make_uint4(sm.x, sm.y, 0u, 0u));
+        const h8 x = *(const h8*)(st.sums + row * st.sp + 32 * at + 8 * u);
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-            const f4v M = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, mv[r], f4v{}, 0, 0, 0);
+            // min_j, 2^-11 min_j and 2^-22 min_j (an exact subnormal) against the parts
+            const uint32_t e = 0x10001000u, m1 = pk_mul(mn[r], e), m2 = pk_mul(m1, e);
+            const h8 mv = __builtin_bit_cast(h8, make_uint4(__builtin_amdgcn_perm(m1, mn[r], 0x05040100u), m2 & 0xFFFFu,
+                                                            __builtin_amdgcn_perm(m1, mn[r], 0x07060302u), m2 >> 16));
+            const f4v M = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, mv, f4v{}, 0, 0, 0);
             const float d = gh_h2f(w[r].hd.x & 0xFFFFu) * 16384.0f, dm = gh_h2f(w[r].hd.x >> 16) * -32.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -298,7 +300,7 @@ __device__ __forceinline__ void few_body(const GhGemmArgs& a, const GhGemmSeg& g
     const uint32_t b0 = z * per, cnt = min(per, nb - b0);  // the host leaves no split empty
     Staged st;
     st.xp = per * 256 + 8;
-    st.sp = per * 16 + 8;
+    st.sp = per * 32 + 8;
     st.xs = lds;
     st.sums = lds + a.n * st.xp;
     // activations: chunk i = 8 values c of token t; the first round is requested ahead of the weights
@@ -328,11 +330,12 @@ __device__ __forceinline__ void few_body(const GhGemmArgs& a, const GhGemmSeg& g
                 s += GH_DPP(s, 0xB1, 0xF);
                 s += GH_DPP(s, 0x4E, 0xF);
                 s *= 0.03125f;
-                const _Float16 hi = (_Float16)s, mid = (_Float16)((s - (float)hi) * 2048.0f);
+                const _Float16 hi = (_Float16)s;
+                const float rest = (s - (float)hi) * 2048.0f;
+                const _Float16 mid = (_Float16)rest, low = (_Float16)((rest - (float)mid) * 2048.0f);
                 if (i < chunks && (tid & 3u) == 0) {
-                    _Float16* sm = lds + a.n * st.xp + t * st.sp + (c >> 5) * 16 + ((c >> 2) & 7u) * 2;
-                    sm[0] = hi;
-                    sm[1] = mid;
+                    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+                    *(h4*)(lds + a.n * st.xp + t * st.sp + (c >> 2) * 4) = h4{hi, mid, low, (_Float16)0.0f};
                 }
             }
         }

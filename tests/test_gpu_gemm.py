@@ -189,6 +189,34 @@ def test_gemm_few_tokens_exact_extremes(hip, fmt, x_scale):
         hip.free_buffer(b)
 
 
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -8, 2.0 ** -15])
+def test_gemm_few_tokens_keeps_the_minima_sums(hip, scale):
+    """Below 8 tokens the sums that the Q4_K minima multiply are FP32 sums, all of whose 24 bits count:
+    weights that are minima alone (quants 0, minima 1), and sub-blocks of activations whose sums
+    32006 + 2^-9 and -32006 leave the last one. Exact in FP32 in any order, so the result is, too."""
+    rows, in_dim, n = 16384, 4096, 3  # 37.7 MB: the few-token kernels, not the GEMV, from 2 tokens
+    block = np.zeros(144, np.uint8)
+    block[2:4] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)  # d = 0, dmin = 1
+    block[8:12] = 1    # minima of sub-blocks 0-3
+    block[12:16] = 16  # and 4-7 (high nibbles)
+    w = np.tile(block, rows * (in_dim // 256))
+    assert (O.dequant(F.FMT_Q4_K, w[:144], 1, 256) == -1.0).all()
+    x = np.zeros((n, in_dim), np.float32)
+    for t in range(n):
+        s0, s1 = 32 * (5 * t), 32 * (5 * t + 3)  # in one block and across two
+        x[t, s0:s0 + 16], x[t, s0 + 20], x[t, s0 + 31] = 2000.0, 6.0, 2.0 ** -9
+        x[t, s1:s1 + 16], x[t, s1 + 20] = -2000.0, -6.0
+    x *= scale
+    a16 = O.f16(x.reshape(-1))
+    assert np.array_equal(O.f32(a16), x.reshape(-1))
+    wb, ab, ob = hip.load_weight(F.FMT_Q4_K, w, in_dim, rows), hip.from_host(a16), hip.alloc_buffer(n * rows * 2)
+    hip.matmul_batched(ob, ab, wb, in_dim, rows, n)
+    got = O.f32(hip.download(ob, np.uint16, n * rows))
+    assert (got == -scale * 2.0 ** -9).all(), np.unique(got)
+    for b in (wb, ab, ob):
+        hip.free_buffer(b)
+
+
 def _lcg(count, seed=0x9E3779B9):
     """The reference test generator, seed = seed * 1664525 + 1013904223 (mod 2^32), as the
     array of its first `count` outputs (blocks of M steps advanced with the M-step map)."""
