@@ -402,7 +402,8 @@ static int attention_prefill(gh_backend* b, GhAttnArgs a, uint32_t group) {
     const uint32_t pq = 16 * rw, nqb = ceil_div(a.rows, pq);
     uint32_t splits = prefill_splits(b, nqb * ng, ceil_div(a.base + a.rows, 64));
     if (splits > 1) {
-        const size_t n = (size_t)a.rows * a.q_heads * splits;
+        // rounded up: the sums are stored 16 bytes at a time (within attention_workspace's slack)
+        const size_t n = ((size_t)a.rows * a.q_heads * splits + 3) / 4 * 4;
         bool room = false;
         const int rc = try_workspace(b, attention_workspace(a.rows, a.q_heads, splits), &room);
         if (rc) return rc;

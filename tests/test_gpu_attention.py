@@ -147,6 +147,27 @@ def test_prefill_attention_non_finite_cache_rows(hip, qh, kvh, base, n):
     _free(hip, qb, ob, kv.k, kv.v)
 
 
+@pytest.mark.parametrize("qh,kvh,n,splits", [(3, 3, 5, 3), (1, 1, 33, 5), (5, 5, 7, 1), (4, 1, 9, 31)])
+def test_prefill_attention_odd_partial_counts(hip, qh, kvh, n, splits):
+    """Key-split partials whose count (rows x heads x splits) is odd, and one that is not a multiple of
+    four: the unnormalized sums start on 16 bytes all the same."""
+    rng = np.random.default_rng(qh + n)
+    base = 2000
+    ctx = base + n
+    kc, vc = (O.f16(rng.standard_normal(ctx * kvh * 128).astype(np.float32)) for _ in range(2))
+    q = O.f16(rng.standard_normal(n * qh * 128).astype(np.float32))
+    kv = _kv(hip, 1, ctx, kvh, kc, vc)
+    qb, ob = hip.from_host(q), hip.alloc_buffer(n * qh * 128 * 2)
+    want = O.f32(O.attention_prefill(q, kc, vc, 128, kvh, qh, base, n, 0, ctx))
+    try:
+        hip.set_attention_splits(splits)
+        hip.attention_prefill(ob, qb, kv, qh, base, n, 0)
+    finally:
+        hip.set_attention_splits(0)
+    _close(O.f32(hip.download(ob, np.uint16, n * qh * 128)), want, "odd")
+    _free(hip, qb, ob, kv.k, kv.v)
+
+
 @pytest.mark.parametrize("qh,kvh", [(8, 8), (16, 8)], ids=["g1", "g2"])
 @pytest.mark.parametrize("gap", [26, 34])
 def test_prefill_attention_long_flat_tail(hip, qh, kvh, gap):
