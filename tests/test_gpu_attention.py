@@ -220,7 +220,7 @@ def _reference_case(ctx_total):
 def test_reference_prefill_attention_vectors(hip, context):
     qh, kc, vc = _reference_case(context)
     kv = _kv(hip, 1, context, 1, kc, vc)
-    for n in (64, 32, 16):  # n = 16 runs the per-row split-K path
+    for n in (64, 32, 16):  # one key-split launch each
         base = context - n
         idx = np.arange(n * qh * 128)
         q = O.f16(((idx % 17).astype(np.float32) * np.float32(0.03) - np.float32(0.22)))
@@ -297,17 +297,19 @@ def test_xcd_probe_confirms_the_mi355x_dispatch():
         assert b.xcd_count == 8
 
 
-@pytest.mark.parametrize("qh,kvh,n", [(12, 3, 7), (64, 8, 5), (32, 8, 20), (16, 16, 3)],
-                         ids=["g4-kv3", "g8", "g4-rows20", "g1-kv16"])
-def test_multi_row_decode_kernels_xcd_grid(hip, qh, kvh, n):
-    """Rows below the matrix-core prefill's minimum (or groups it does not serve) run the
-    decode kernels with several query rows. In the XCD-local grid the (row, kv head) pairs fill
+@pytest.mark.parametrize("qh,kvh,n,base", [(12, 3, 7, 600), (64, 8, 5, 600), (32, 8, 20, 600), (16, 16, 3, 600),
+                                           (8, 1, 6, 600), (4, 1, 20, 600), (16, 16, 3, 300), (6, 3, 8, 600)],
+                         ids=["g4-kv3", "g8", "g4-rows20", "g1-kv16", "g8-kv1", "g4-kv1-rows20", "g1-kv16-near", "g2-kv3"])
+def test_multi_row_decode_kernels_xcd_grid(hip, qh, kvh, n, base):
+    """A few rows over little cache (rows x positions x kv heads up to 16384, 4096 with eight query
+    heads per kv head: the first case and the last four) run the decode kernels with several query
+    rows, the others the prefill kernels, which the merge form does not touch. In the XCD-local grid the (row, kv head) pairs fill
     z-groups of xcds, the last one partly (kv_heads 3: 21 pairs): both merge forms give the
     same bits, within the oracle bar, at every split count the row lengths allow."""
     if not hip.xcd_count:
         pytest.skip("dispatch placement not confirmed on this device")
     rng = np.random.default_rng(qh * 7 + kvh + n)
-    ctx, base = 1024, 600
+    ctx = 1024
     kc = O.f16(rng.standard_normal(ctx * kvh * 128).astype(np.float32))
     vc = O.f16(rng.standard_normal(ctx * kvh * 128).astype(np.float32))
     q = O.f16(rng.standard_normal(n * qh * 128).astype(np.float32))

@@ -1,4 +1,4 @@
-"""Matrix-core prefill GEMM (gh_matmul_batched with n >= 8 tokens) against the oracle.
+"""Matrix-core prefill GEMM (gh_matmul_batched with several tokens) against the oracle.
 
 Bars:
   * kernel arithmetic: against an fp64 product of the FP16-rounded reference-dequantized
@@ -110,7 +110,7 @@ def test_gemm_c3_full_size(hip, fmt, rows, in_dim):
 
 
 def test_gemm_equals_gemv_within_tolerance_at_threshold(hip):
-    """n = 7 runs the GEMV (exact quant arithmetic), n = 8 the GEMM (FP16 weight tiles): each
+    """n = 7 of a matrix this small runs the GEMV (exact quant arithmetic), n = 8 the GEMM (FP16-rounded weights): each
     meets the fp64 bar of its own operands on the same data."""
     fmt, rows, in_dim = F.FMT_Q4_K, 256, 2048
     rng = np.random.default_rng(99)

@@ -296,6 +296,34 @@ def test_rope_batched_widths(hip, rope_dim, heads, kheads, rows, shift):
         hip.free_buffer(buf)
 
 
+@pytest.mark.parametrize("rope_dim,heads,kheads,rows,base", [(128, 4, 2, 40, 16360), (128, 7, 3, 9, 100000),
+                                                              (10, 3, 1, 9, 40000)])
+def test_rope_batched_post_scale(hip, rope_dim, heads, kheads, rows, base):
+    """Past position 16384 the queries' post-scale is not 1: it reaches every query head and no key
+    head of the one launch, in both access widths. Keys: the oracle's bits. Queries: the kernel rounds
+    the product with the post-scale to FP16 once, where the oracle rounds it to FP32 first, so
+    a value next to an FP16 tie may be the neighbour (about one in 10^5)."""
+    rng = np.random.default_rng(rope_dim + rows)
+    q, k = (O.f16(rng.standard_normal(rows * h * 128).astype(np.float32)) for h in (heads, kheads))
+    qb, kb = hip.from_host(q), hip.from_host(k)
+    oy = O.Yarn(rope_dim, 16384, 1e6, 16.0, 32.0, 1.0, 1.0, 0.1)
+    hip.rope_yarn_batched(qb, kb, heads, kheads, 128, base, rows, replace(YARN, rope_dim=rope_dim))
+    for buf, src, h, role in ((qb, q, heads, F.ROPE_QUERY), (kb, k, kheads, F.ROPE_KEY)):
+        got, want, other = hip.download(buf, np.uint16, len(src)), src.copy(), src.copy()
+        for r in range(rows):
+            a = r * h * 128
+            want[a:a + h * 128] = O.rope_yarn(src[a:a + h * 128], h, 128, base + r, oy, role)
+            other[a:a + h * 128] = O.rope_yarn(src[a:a + h * 128], h, 128, base + r, oy, F.ROPE_QUERY + F.ROPE_KEY - role)
+        # the roles differ here, in nearly every rotated value of the rows past 16384 (16 of 40 in the first case)
+        assert np.mean(want != other) > 0.9 * rope_dim / 128 * np.mean(base + np.arange(rows) >= 16384)
+        if role == F.ROPE_KEY:
+            assert np.array_equal(got, want)
+        else:
+            assert (np.abs(got.astype(np.int32) - want.astype(np.int32)) <= 1).all()  # neighbours of one sign
+            assert np.mean(got != want) <= 1e-3
+        hip.free_buffer(buf)
+
+
 def test_residual_add_bit_exact(hip):
     rng = np.random.default_rng(7)
     n = 5120
@@ -537,8 +565,8 @@ def test_model_prefill_matches_oracle(hip):
 
 @pytest.mark.parametrize("n", [8, 32, 128])
 def test_model_prefill_short_chunk_matches_oracle(hip, n):
-    """A prompt of n rows in one chunk (8: the smallest GEMM batch; 32; 128: one full 128-token
-    tile) on the small shape (the down GEMM splits K, its residual tail summing the splits),
+    """A prompt of n rows in one chunk (8: the fewest over FP16-rounded weights; 32: the few-token
+    kernels, too; 128: one full 128-token tile) on the small shape (the down GEMM splits K, its residual tail summing the splits),
     against the oracle's prefill of the same prompt: the logits and every K/V cache row the
     chunk wrote."""
     shape, ctx = synth.SHAPES["small"], 160
@@ -665,16 +693,18 @@ def test_fused_decode_is_bit_identical_to_op_by_op(hip, shape_name):
 @pytest.mark.parametrize("n", [8, 37, 128, 300])
 @pytest.mark.parametrize("shape_name", ["tiny", "small"])
 def test_prefill_driver_is_bit_identical_to_op_by_op(hip, shape_name, n):
-    """The driver's prefill (one batch: GEMV for n < 8 rows, the MFMA GEMMs above, the
-    warp-specialized ones from 256 rows, with the glue folded into GEMM epilogues and split
-    reduces and Q/K/V in one launch) leaves the same logits and KV bits as recording every
-    trait op separately (prefill::record_batch over the C ABI). The tiny shape's GEMMs run one
-    K split each; the small shape's run one (two for down) at 8-128 rows and two (four for
-    down) at 300, alike in the fused and the separate launches, so both sum in the same order.
-    At 8-128 rows the driver's gate and up run as one paired launch (gh_gemm3_swiglu_r96_t128:
-    48 gate + 48 up rows per tile, silu_mul in its epilogue; 22 and 43 tiles here, the last one
-    partial) against two unsplit GEMMs and silu_mul op by op; at 300 rows they share one split
-    reduce that applies silu_mul (gh_gemm_reduce_swiglu). Where the split counts differ
+    """The driver's prefill (one batch from 8 rows: the few-token kernels up to 48, the tiles above,
+    with the glue folded into GEMM epilogues and split reduces and Q/K/V in one launch) leaves the same
+    logits and KV bits as recording every trait op separately (prefill::record_batch over the C
+    ABI; below 8 rows, where the separate operations run the GEMV for matrices of this size, see
+    test_full_width_short_chunk_over_a_filled_cache). At 8 and 37 rows every matrix runs in splits of
+    two 256-column blocks (tiny: one split, two for down; small: two and four), whichever launch it is
+    in. At 128 the tiny shape's GEMMs run one K split each and the small shape's one (two for
+    down), at 300 two (four for down), alike in the fused and the separate launches, so both sum in the
+    same order. At 128 rows the driver's gate and up run as one paired launch
+    (gh_gemm3_swiglu_r96_t128: 48 gate + 48 up rows per tile, silu_mul in its epilogue; 22 and 43 tiles
+    here, the last one partial) against two unsplit GEMMs and silu_mul op by op; at 8, 37 and 300 rows they
+    share one split reduce that applies silu_mul (gh_gemm_reduce_swiglu). Where the split counts differ
     (the 8B shape's Q/K/V launch against the three projections alone) the results differ only
     by FP32 re-association, checked against the oracle in test_gpu_model_shapes."""
     from graph_horizon_amd import HipModel
