@@ -181,8 +181,8 @@ def main():
                          "hipBLASLt) at the C3 shapes beside this build's dequantizing GEMMs, "
                          "same box, same timing")
     ap.add_argument("--probe-tokens", type=int, default=512,
-                    help="token rows of --gemm-probe's GEMMs (512: the C3 shape; 8-128 run the "
-                         "128-token tiles)")
+                    help="token rows of --gemm-probe's GEMMs (512: the C3 shape; 2-48 run the "
+                         "few-token kernels, 49-128 the 128-token tiles)")
     ap.add_argument("--probe-bytes", default="9437184,94371840",
                     help="comma-separated read sizes for --floor-probe")
     ap.add_argument("--probe-groups", default="256,512,1024,2048",

@@ -226,7 +226,8 @@ class HipBackend:
         self._ok(self.lib.gh_set_scratch_limit(self.h, nbytes), "set_scratch_limit")
 
     def set_attention_splits(self, splits: int):
-        """Decode attention workgroups per (row, kv head); 0 = the backend's policy."""
+        """Decode attention workgroups per (row, kv head) and key splits of prefill attention's
+        16-row query blocks; 0 = the backend's policy."""
         self._ok(self.lib.gh_set_attention_splits(self.h, splits), "set_attention_splits")
 
     def set_attention_xcd_merge(self, enable: bool):

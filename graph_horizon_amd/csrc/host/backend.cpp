@@ -90,8 +90,8 @@ const KernelName kKernels[] = {
 const char* kModules[] = {"gh_quant", "gh_gemv", "gh_glue", "gh_attention", "gh_gemm", "gh_gemm_few"};
 
 constexpr uint32_t kArgmaxBlocks = 256;
-// argmax scratch at the front of the workspace: f32[256] values, u32[256] indices, u32 result
-constexpr size_t kArgmaxBytes = 256 * 4 * 2 + 256;
+// argmax scratch at the front of the workspace: f32[256] values, u32[256] indices
+constexpr size_t kArgmaxBytes = 256 * 4 * 2;
 constexpr size_t kResultBytes = 2 * 128 * 4;  // read_argmax's index, or read_topk's 128 indices and values
 
 std::string library_dir() {
@@ -344,7 +344,8 @@ int op_kv_write(gh_backend* b, const gh_kv* kv, const gh_buf* k, const gh_buf* v
 // workgroups per CU, at most one per 64-position chunk and at most 32 (the merge's limit);
 // longer contexts loop over chunks. (Eight-wave workgroups over 128-position chunks measured
 // 35.5 vs 37.1 us at ctx 32768 but 613 vs 625 tok/s on the 8B decode: not kept.)
-// gh_set_attention_splits replaces the policy's count (still capped by chunks and 32).
+// gh_set_attention_splits replaces the policy's count (still capped by chunks and 32; prefill
+// launches by prefill_splits).
 uint32_t attention_splits(const gh_backend* b, uint32_t max_len, uint32_t kv_heads, uint32_t rows) {
     const uint32_t chunks = ceil_div(max_len, 64);
     const uint32_t want = b->attn_splits ? b->attn_splits
@@ -585,7 +586,7 @@ int op_argmax(gh_backend* b, const gh_buf* logits, uint64_t vocab, void* out, vo
     a.logits = logits->addr;
     a.part_v = (uint64_t)b->ws;
     a.part_i = (uint64_t)((char*)b->ws + 1024);
-    a.out = out ? (uint64_t)out : (uint64_t)((char*)b->ws + 2048);
+    a.out = (uint64_t)out;
     a.out2 = (uint64_t)out2;
     a.step_scalars = (uint64_t)step_scalars;
     a.step_history = (uint64_t)step_history;
@@ -1680,8 +1681,8 @@ int gh_read_argmax(gh_backend* b, const gh_buf* logits, uint64_t vocab, uint32_t
 }
 
 // read_topk: k <= 128 on the device (gh_topk_partial over stripes of at most kTopkChunk
-// logits per step, at most 128 stripes, then gh_topk_final; 8 k bytes come back), larger k
-// on the host over the read-back logits. Both give exactly the reference's selection and
+// logits per step, at most kTopkStripes stripes, then gh_topk_final, which leaves 8 k bytes in pinned
+// host memory), larger k on the host over the read-back logits. Both give exactly the reference's selection and
 // order (cpu/readback.rs:59-69): (logit desc by f32 total order, index asc).
 constexpr uint64_t kTopkDeviceMax = 128, kTopkChunk = 512, kTopkStripes = 256;
 

@@ -260,8 +260,6 @@ int op_gemv(gh_backend* b, const GemvSeg* segs, uint32_t nseg, const gh_buf* x, 
 // (out = silu_mul(gate, f16(acc))). resid != 0: the output row is folded into the FP32 residual
 // x[n][out_dim] (residual_add) and, with norm != 0, its RMSNorm written to normed — the bits of
 // the separate reduce, residual_add and rmsnorm_x ops (out then only holds the FP16 projection).
-// rope != nullptr: the output rows (query or key heads of head_dim) are rotated at positions
-// base + t as op_rope does — in the split reduce, or by op_rope after an unsplit GEMM.
 struct GemmEpi {
     uint32_t epi = GH_GEMM_EPI_F16;
     uint64_t aux = 0;
@@ -281,16 +279,18 @@ int op_gemm_swiglu(gh_backend* b, const gh_buf* out, const gh_buf* gate, const g
 int op_matmul_epi(gh_backend* b, const gh_buf* out, const gh_buf* a, const gh_buf* w, uint32_t in_dim,
                   uint32_t out_dim, uint32_t n, const gh_buf* gate, const gh_buf* resid,
                   const gh_buf* norm = nullptr, const gh_buf* normed = nullptr, float eps = 0.0f);
+// Whether an out_dim-row output of n >= 2 tokens can be given a RoPE role (whole heads).
 bool gemm_rope_applies(uint32_t n, uint32_t out_dim, uint32_t head_dim, const GhRopeTable& rope);
 // Batches of more than 128 tokens run the GEMMs in 256-token tiles, over a registered FP16 copy
 // of the weights (b->w16) where there is one; 128 tokens or fewer fit the 128-token tiles of
 // the dequantizing kernels exactly, where a copy's four-fold weight stream costs more. Both
 // forms of a batch size share one tile and split plan, so they give the same bits.
 constexpr uint32_t kGemmTallTokens = 129;
-// Several projections of one FP16 input (n >= 2 tokens) in one warp-specialized launch (row
-// tiles of 128, each in its matrix's format) and one split reduce that writes each matrix's
+// Several projections of one FP16 input (n >= 2 tokens) in one launch (few-token or warp-specialized,
+// row tiles of 128 or 256, each in its matrix's format) and one split reduce that writes each matrix's
 // FP16 output and applies its RoPE role (GH_GEMM_ROLE_*; rows of head_dim, positions base + t)
-// — the values of separate gh_matmul_batched launches and op_rope.
+// — the values of op_gemm per matrix and op_rope, up to the order of the sums where the launch
+// splits K differently.
 struct GemmSegSpec {
     const gh_buf* w;
     const gh_buf* out;
@@ -299,8 +299,6 @@ struct GemmSegSpec {
 bool gemm_multi_applies(uint32_t n);
 int op_gemm_multi(gh_backend* b, const gh_buf* a, const GemmSegSpec* segs, uint32_t nseg, uint32_t n,
                   const GhRopeTable* rope, uint32_t base, uint32_t head_dim);
-// gh_matmul_batched then op_rope(role, positions base + t) on its output, the rotation folded
-// into the split reduce when the GEMM splits K (n >= 2 tokens, out_dim a multiple of head_dim).
 size_t attention_workspace(uint32_t rows, uint32_t q_heads, uint32_t splits);
 uint32_t attention_splits(const gh_backend* b, uint32_t max_len, uint32_t kv_heads, uint32_t rows);
 int ensure_counters(gh_backend* b, size_t slots);

@@ -223,8 +223,10 @@ bool fusable(const gh_model* m, uint32_t li) {
 // epilogues carry the glue: the O and down projections' output rows go straight into the
 // residual and the following RMSNorm (gh_gemm_tail), silu_mul is applied in the gate and up
 // projections' shared split reduce (or the up projection's epilogue); *normed on return says
-// the next layer's attention norm is already in s.normed. The values are those of the
-// separate ops below.
+// the next layer's attention norm is already in s.normed. From 8 rows the values are those of the
+// separate ops below (up to the order of FP32 sums where a launch splits K differently). At 2 to 7 rows
+// both sides multiply exact weights, but the separate ops of matrices small enough run the GEMV and
+// the driver always the few-token kernels, so a few FP16 results are the neighbouring value.
 int layer(gh_model* m, gh_encoder* enc, const Scratch& s, uint32_t li, uint32_t base,
           uint32_t rows, const void* pos_ptr, bool* normed = nullptr) {
     if (rows == 1 && fusable(m, li)) return layer_decode_fused(m, enc, s, li, base, pos_ptr);

@@ -407,7 +407,7 @@ __device__ __forceinline__ TopkList<V> topk_lists(const P src, uint32_t first, u
 }
 
 // One workgroup of 16 waves merges the stripes' lists, 16 apart per wave, then one wave the 16 lists
-// left, and writes k (u32 index, f32 bits) pairs.
+// left, and writes k u32 indices, then their f32 bits.
 template <int V>
 __device__ __forceinline__ void topk_final(const GhTopkArgs& a, uint64_t* s) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;

@@ -208,7 +208,10 @@ int gh_timer_stop(gh_backend* b, float* ms);
 int gh_synchronize(gh_backend* b);
 /* Attention split count (no counterpart in the reference: a test and tuning hook). Decode
  * attention splits each (row, kv head) over this many workgroups (at most one per 64-position
- * chunk); 0 restores the backend's policy (about two workgroups per CU). At most 32. Graphs
+ * chunk); 0 restores the backend's policy (about two workgroups per CU). Prefill attention
+ * splits the keys of its 16-row query blocks over as many (at most one per 64-key tile; launches
+ * whose 32-row blocks fill the CUs stay unsplit), where the policy splits only if the blocks leave CUs
+ * idle. A split count changes the order of FP32 sums, so the outputs' last bits. At most 32. Graphs
  * recorded before the call are re-recorded on their next use. */
 int gh_set_attention_splits(gh_backend* b, uint32_t splits);
 /* Decode attention's split merge (no counterpart in the reference: a test and tuning hook).
